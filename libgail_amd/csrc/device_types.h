@@ -8,6 +8,13 @@ namespace gail_amd {
 constexpr int kMaxPasses = 64;       // pass table capacity per code-block
 constexpr int kMaxPlanes = 24;       // magnitude bit-planes a code-block can carry
 constexpr int kPlaneSymCap = 2560;   // symbols one bit-plane of a 32x32 block can produce
+// A plane's symbols as the MQ coder reads them (context << 1 | bit): each pass filled up to a
+// whole 4-byte word (one at least) with neutral symbols and the top bit of its last symbol set,
+// each plane filled up to whole 16-byte groups. Neutral symbols have a context of their own in
+// which coding changes nothing.
+constexpr int kPlaneStage = kPlaneSymCap + 32;
+constexpr uint32_t kSymPad = 19u << 1, kSymPassEnd = 0x80u;
+constexpr int kMqContexts = 20;
 constexpr uint32_t kLog2Max = 2560;  // counts the entropy-estimate table covers
 
 // One code-block of a job (16 bytes). coef_off is the float index of the block's
@@ -43,11 +50,11 @@ struct T1Info {
     uint32_t symbols;  // total symbols
 };
 
-// MQ coder state at the end of a pass (16 bytes).
+// MQ coder state at the end of a pass (16 bytes), as the coder holds it: bytes may still be
+// in the code register (t1_mq_kernel).
 struct MqSnapshot {
-    int32_t bp;       // index of the pending byte (-1 before the first byte)
-    uint32_t b_ct;    // pending byte | CT << 16
-    uint32_t c, a;
+    uint32_t bp_b_d;         // (index of the pending byte + 1) << 16 | pending byte << 8 | shifts left + 16
+    uint32_t c_lo, c_hi, a;  // code register, interval << 16
 };
 
 // Counters of a job, cleared by a kernel before each run (never by a memset node).

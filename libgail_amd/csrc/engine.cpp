@@ -163,7 +163,7 @@ size_t Job::estimateBytes(const std::vector<SlotCapacity>& slots, const JobOptio
         lv = std::max(lv, lim.levels);
     }
     const Sizes z = t1Sizes(coefs, n, opt.poolBytesPerCoef);
-    total += (size_t)n * (16 + 16 + 3 * kMaxPasses * 4 + kMaxPlanes * 8 + kMaxPasses * 16 + 4 + 8 + 8 + 4);
+    total += (size_t)n * (16 + 16 + 2 * kMaxPasses * 4 + kMaxPlanes * 8 + kMaxPasses * 16 + 4 + 8 + 8 + 4);
     total += (size_t)nb * sizeof(T1Band) + (size_t)lv * slots.size() * sizeof(DwtLevelDesc);
     // device rate control: hull points and their slope bins, chosen passes, slope ranges,
     // one histogram per slot
@@ -317,7 +317,6 @@ void Job::allocate() {
 
     const uint32_t n = blockCap_;
     dInfo_ = devAlloc<T1Info>(n);
-    dPassEnd_ = devAlloc<uint32_t>((size_t)n * kMaxPasses);
     dPassDist_ = devAlloc<int32_t>((size_t)n * kMaxPasses);
     dPassLen_ = devAlloc<uint32_t>((size_t)n * kMaxPasses);
     dChunks_ = devAlloc<uint2>((size_t)n * kMaxPlanes);
@@ -715,10 +714,6 @@ void Job::uploadAsync(int i) {
     hipCheck(hipMemcpyAsync(sd_[i].in, hostInput(i), sd_[i].inBytes, hipMemcpyHostToDevice, stream_), "frame upload");
 }
 
-// Launches of at most this many blocks code their longest blocks one per wave: with a
-// batch's worth of blocks the lane waves fill the machine and the scalar coder only competes.
-constexpr uint32_t kMqUniformMaxBlocks = 65536;
-
 void Job::enqueueT1(hipStream_t s) {
     const uint32_t n = nblocks_;
     hipCheck(launch_clear_counters(dCounters_, dWork_, 4, s), "clear counters");
@@ -729,7 +724,6 @@ void Job::enqueueT1(hipStream_t s) {
     cm.nblocks = n;
     cm.max_passes = kMaxPasses;
     cm.info = dInfo_;
-    cm.pass_end = dPassEnd_;
     cm.pass_dist = dPassDist_;
     cm.chunks = dChunks_;
     cm.pool = dPool_;
@@ -747,7 +741,6 @@ void Job::enqueueT1(hipStream_t s) {
     hipCheck(launch_out_offsets(dInfo_, n, dOutOff_, dPartial_, s), "codeword offsets");
     MqParams mq{};
     mq.info = dInfo_;
-    mq.pass_end = dPassEnd_;
     mq.chunks = dChunks_;
     mq.pool = dPool_;
     mq.perm = dPerm_;
@@ -760,10 +753,14 @@ void Job::enqueueT1(hipStream_t s) {
     mq.counters = dCounters_;
     mq.nblocks = n;
     mq.work_next = dWork_ + 1;
-    mq.nlong = n <= kMqUniformMaxBlocks ? std::min<uint32_t>(n, (uint32_t)(ctx_.computeUnits() * opt_.mqLongPerCU)) : 0u;
-    // enough waves for one long block each, where the grid cap allows
+    // One wave per SIMD where the blocks do not fill 64-lane waves: a wave's time is that of its
+    // longest block, and fewer blocks in it take fewer slow steps in common (one 4K frame, 26
+    // blocks per wave: 1.63 ms, 64: 1.74; a 512x256 frame, 1 per wave: 1.24 ms, 64: 1.55). Two
+    // waves per SIMD are no better (1.72 ms with 13): the steps fill the issue slots.
+    const uint32_t simds = (uint32_t)ctx_.computeUnits() * 4;
+    mq.lanes = std::min<uint32_t>(64, (n + simds - 1) / simds);
     const uint32_t mqWaves = (uint32_t)opt_.mqGroup / 64;
-    const uint32_t mqWant = std::max<uint32_t>((n + opt_.mqGroup - 1) / opt_.mqGroup, (mq.nlong + mqWaves - 1) / mqWaves);
+    const uint32_t mqWant = (n + mq.lanes * mqWaves - 1) / (mq.lanes * mqWaves);
     const int mqGroups = (int)std::max<uint32_t>(
         1, std::min<uint32_t>(mqWant, (uint32_t)(ctx_.computeUnits() * opt_.mqGroupsPerCU)));
     hipCheck(launch_t1_mq(mq, opt_.mqGroup, opt_.mqRead, mqGroups, s), "MQ coding");

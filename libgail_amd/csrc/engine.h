@@ -44,7 +44,6 @@ struct JobOptions {
     int mqGroup = 256;        // MQ workgroup size
     int mqRead = 64;          // symbol bytes each MQ lane reads at a time (16 or 64)
     int mqGroupsPerCU = 8;
-    int mqLongPerCU = 8;      // longest blocks per compute unit coded one per wave
     double poolBytesPerCoef = 8.0;  // symbol pool sizing (grown on overflow)
     bool useGraph = false;    // replay the launch chain as a HIP graph
 };
@@ -302,7 +301,6 @@ private:
     uint32_t* dRcHist_ = nullptr;
     // Tier-1 arrays
     T1Info* dInfo_ = nullptr;
-    uint32_t* dPassEnd_ = nullptr;
     int32_t* dPassDist_ = nullptr;
     uint32_t* dPassLen_ = nullptr;
     uint2* dChunks_ = nullptr;

@@ -46,9 +46,8 @@ struct CmParams {
     uint32_t nblocks;
     uint32_t max_passes;
     T1Info* info;
-    uint32_t* pass_end;   // [block][64] cumulative symbol counts
     int32_t* pass_dist;   // [block][64]
-    uint2* chunks;        // [block][24]: (offset / 16, count) of each bit-plane's symbols
+    uint2* chunks;        // [block][24]: (offset / 16, bytes) of each bit-plane's symbols
     uint8_t* pool;
     unsigned long long pool_cap;
     JobCounters* counters;
@@ -58,7 +57,6 @@ struct CmParams {
 
 struct MqParams {
     const T1Info* info;
-    const uint32_t* pass_end;
     const uint2* chunks;
     const uint8_t* pool;
     const uint32_t* perm;
@@ -71,7 +69,7 @@ struct MqParams {
     JobCounters* counters;
     uint32_t nblocks;
     uint32_t* work_next;
-    uint32_t nlong;                     // leading blocks of perm coded one per wave (<= nblocks)
+    uint32_t lanes;                     // blocks a wave codes at a time (1..64)
 };
 
 struct CompactParams {

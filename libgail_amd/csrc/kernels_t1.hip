@@ -13,9 +13,10 @@
 // LDS staging buffer, copied to an HBM pool once per bit-plane.
 //
 // MQ coding: one lane per code-block, blocks ordered largest first so a wave's lanes
-// finish together. The coder keeps A, C, CT and the pending byte in registers and the 19
-// context states in LDS; at each pass end it snapshots its state, and after the final
-// flush it derives every pass's truncation length from the snapshots.
+// finish together. The coder keeps A, C, CT and the pending byte in registers, with several
+// bytes' room in C so that bytes are taken rarely and for all lanes at once, and the context
+// states in LDS; at each pass end it snapshots its state, and after the final flush it derives
+// every pass's truncation length from the snapshots.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -142,7 +143,7 @@ template <int WAVES>
 __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
     // a plane's symbols per block, then 128 bytes where each lane writes the symbols its rows
     // do not have (so that every lane stores on every step)
-    __shared__ __attribute__((aligned(16))) uint8_t s_sym[WAVES][2][kPlaneSymCap + 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_sym[WAVES][2][kPlaneStage + 128];
     // Early-termination counts per context of the current plane (d = 0 low half, d = 1 high
     // half) and the contexts' entropy terms.
     __shared__ uint32_t s_hist[WAVES][2][32];
@@ -150,7 +151,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
 
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, half = lane >> 5, x = lane & 31;
     uint8_t* const sym = s_sym[wv][half];
-    uint8_t* const junk = sym + kPlaneSymCap + 4 * x;
+    uint8_t* const junk = sym + kPlaneStage + 4 * x;
     uint32_t* const hist = s_hist[wv][half];
     float* const terms = s_term[wv][half];
     unsigned long long chunk_cur = 0, chunk_end = 0;  // wave-uniform sub-allocator
@@ -247,6 +248,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
             int plane_dist = 0;
             for (int type = (j == 0 ? 2 : 0); type < 3; ++type) {
                 const bool pact = act && np < P.max_passes;
+                const uint32_t pass_start = plane_count;
                 const uint32_t colMask = (pact && x < w) ? rowsValid : 0u;
                 const uint32_t SL = from_left(S, x), SR = from_right(S, x);
                 // The pass over the whole column: keep0 the rows whose zero-coding (or
@@ -389,19 +391,30 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                             }
                         }
                     }
+                    sym_total += base - plane_count;
                     plane_count = base;
                 }
                 const int total = half_total(dist);
                 if (pact) {
+                    // the pass ends a 4-byte word of the MQ coder's input, the word's top bit set
+                    const uint32_t pad = plane_count == pass_start ? 4u : (0u - plane_count) & 3u;
+                    if ((uint32_t)x < pad) sym[plane_count + x] = (uint8_t)kSymPad;
+                    plane_count += pad;
                     if (x == 0) {
-                        P.pass_end[(size_t)cb * kMaxPasses + np] = sym_total + plane_count;
+                        sym[plane_count - 1] |= (uint8_t)kSymPassEnd;
                         P.pass_dist[(size_t)cb * kMaxPasses + np] = total;
                     }
                     ++np;
                     plane_dist += total;
                 }
             }
-            // ---- the plane's symbols to the pool (wave-uniform sub-allocation)
+            // ---- the plane's symbols to the pool (wave-uniform sub-allocation), filled up to
+            // whole 16-byte groups with neutral symbols
+            {
+                const uint32_t fill = (16u - (plane_count & 15u)) & 15u;
+                if ((uint32_t)x < fill) sym[plane_count + x] = (uint8_t)kSymPad;
+                plane_count += fill;
+            }
             wave_sync();
             // early-termination counts of the plane's symbols, 32 lanes per block at a time
             // (not one lane per column inside the divergent emission loops)
@@ -411,8 +424,8 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
 #pragma unroll
                     for (uint32_t j = 0; j < 4; ++j)
                         if (i + j < plane_count) {
-                            const uint32_t sv = (w4 >> (8 * j)) & 0xFFu;
-                            atomicAdd(&hist[sv >> 1], (sv & 1u) ? 0x10000u : 1u);
+                            const uint32_t sv = w4 >> (8 * j);
+                            atomicAdd(&hist[(sv >> 1) & 31u], (sv & 1u) ? 0x10000u : 1u);
                         }
                 }
             const uint32_t cnt_lo = __shfl((int)plane_count, 0), cnt_hi = __shfl((int)plane_count, 32);
@@ -435,10 +448,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                     *(uint4*)(P.pool + off + i) = *(const uint4*)(sym + i);
                 if (x == 0) P.chunks[(size_t)cb * kMaxPlanes + j] = make_uint2((uint32_t)(off >> 4), plane_count);
             }
-            if (act) {
-                sym_total += plane_count;
-                ++planes;
-            }
+            if (act) ++planes;
             wave_sync();
             // ---- early termination after plane p > 0 (t1_ref.cpp:128-162)
             bool stop_now = false;
@@ -719,39 +729,77 @@ hipError_t launch_compact_offsets(const T1Info* info, const uint32_t* code_len, 
 
 // ---------------------------------------------------------------- MQ coding
 namespace {
-// Table C.2 packed as Qe | NMPS << 16 | NLPS << 22 | SWITCH << 28. A context's state word is
-// its entry of this table with its MPS in bit 31.
-__constant__ uint32_t kMqTable[47];
+// The coder's states (t1_tables.h: build_mq_coder_table).
+__constant__ uint32_t kMqTable[2 * kMqCoderStates];
+__constant__ uint32_t kMqInitial[4];  // contexts start in states 0, 4 (zero coding 0), 3 (run length), 46 (uniform)
 
 }  // namespace
 
+// The MQ encoder (C.2) with its byte-outs put off. The code register L holds C << 5 in 64
+// bits: bits 5-31 are the 27 bits below the carry, bit 32 is the carry into the pending byte B,
+// and whatever has been shifted past it are bytes that BYTEOUT (C.2.7) has not taken yet. D is
+// CT + 16, so BYTEOUT is due when D <= 16 and must run before D would fall below -15.
+//
+// Taking bytes late gives the same bytes as taking them at once, except where an addition
+// carries into a byte of 0xFF that is due but not taken: a byte of 0xFF takes no carry, which
+// goes to the bit stuffed after it. Such a carry passes bit 31 on its way up, so the caller
+// takes every byte that is due before it makes an addition that carries out of bit 31.
+struct MqCode {
+    uint64_t L;
+    int32_t D;
+    uint32_t B;
+    int32_t bp;  // index of the pending byte
+
+    // BYTEOUT, due (D <= 16): returns the byte at bp, final, and the next one becomes pending;
+    // the caller counts bp on.
+    __device__ __forceinline__ uint32_t byteout() {
+        const int sh = 40 - D;
+        const uint32_t X = (uint32_t)(L >> sh);  // carry and the 8 bits of the byte due
+        const uint32_t carry = B != 0xFFu ? X >> 8 : 0u;
+        const uint32_t byte = B + carry;
+        const uint32_t stuff = byte == 0xFFu ? 1u : 0u;
+        L -= (uint64_t)(X & ~stuff) << sh;
+        B = (X - (carry << 8)) >> stuff;
+        D += 8 - (int)stuff;
+        return byte;
+    }
+};
+
 // Truncation length of every pass but the last (mq_encoder.h:146-169): the shortest prefix,
 // never ending in 0xFF, that with the decoder's 1-fill stays inside the interval the coder had
-// at the pass end. out holds the block's len codeword bytes.
-__device__ __forceinline__ void mq_pass_lengths(const uint8_t* out, uint32_t len, const MqSnapshot* snaps,
+// at the pass end. out holds the block's len codeword bytes, readable to cap (a multiple of 64).
+// At most 6 bytes decide a pass: they are read at once, the next snapshot one pass ahead.
+__device__ __forceinline__ void mq_pass_lengths(const uint8_t* out, uint32_t len, uint32_t cap, const MqSnapshot* snaps,
                                                 uint32_t np, uint32_t* plen) {
     uint32_t prev = 1;
+    MqSnapshot next = snaps[0];
     for (uint32_t q = 0; q + 1 < np; ++q) {
-        const MqSnapshot sn = snaps[q];
-        const int ct = (int)(sn.b_ct >> 16);
-        const int base_sh = 43 - ct;
-        const unsigned long long low =
-            ((unsigned long long)(sn.b_ct & 0xFFFFu) << base_sh) + ((unsigned long long)sn.c << 16);
-        const unsigned long long high = low + ((unsigned long long)sn.a << 16);
+        const MqSnapshot sn = next;
+        next = snaps[q + 1];
+        MqCode m{((uint64_t)sn.c_hi << 32) | sn.c_lo, (int32_t)(sn.bp_b_d & 0xFFu), (sn.bp_b_d >> 8) & 0xFFu,
+                 (int32_t)(sn.bp_b_d >> 16) - 1};
+        for (; m.D <= 16; ++m.bp) m.byteout();
+        const uint32_t at = m.bp < 0 ? 0u : (uint32_t)m.bp, g = at & ~7u, r = 8u * (at & 7u);
+        const uint64_t g0 = g < cap ? *(const uint64_t*)(out + g) : 0ull;
+        const uint64_t g1 = g + 8u < cap ? *(const uint64_t*)(out + g + 8u) : 0ull;
+        uint64_t bytes = (g0 >> r) | ((g1 << 1) << (63u - r));
+        if (m.bp < 0) bytes <<= 8;  // the dummy byte
+        const int base_sh = 43 - (m.D - 16);
+        const unsigned long long low = ((unsigned long long)m.B << base_sh) + (m.L << 11);
+        const unsigned long long high = low + sn.a;
         unsigned long long prefix = 0;
-        int rel = 0;
+        int sh = base_sh;
         uint32_t L = len;
-        for (int i = sn.bp; i < (int)len; ++i) {
-            const uint32_t byte = i >= 0 ? out[i] : 0u;
-            const int sh = base_sh - rel;
-            if (sh < 0) break;
+        for (int i = m.bp; i < (int)len && sh >= 0; ++i) {
+            const uint32_t byte = (uint32_t)bytes & 0xFFu;
+            bytes >>= 8;
             prefix += (unsigned long long)byte << sh;
             const unsigned long long tail = prefix + (1ull << sh);
             if ((uint32_t)(i + 1) >= prev && byte != 0xFFu && tail <= high && tail > low) {
                 L = (uint32_t)(i + 1);
                 break;
             }
-            rel += byte == 0xFFu ? 7 : 8;
+            sh -= byte == 0xFFu ? 7 : 8;
         }
         plen[q] = L;
         prev = L > prev ? L : prev;
@@ -759,170 +807,47 @@ __device__ __forceinline__ void mq_pass_lengths(const uint8_t* out, uint32_t len
     plen[np - 1] = len;
 }
 
-// One code-block coded by a whole wave, for the longest blocks of a launch: a lane-per-block
-// wave advances all its blocks one symbol per step of about a hundred instructions, so its
-// longest block sets the launch's time. Here the coder's registers are wave-uniform (scalar)
-// values, the 19 context states sit in lanes 0-18 of one vector register and Table C.2 in
-// lanes 0-46 of another (tabv), both read with readlane, and a symbol is a short chain of
-// scalar instructions. The bytes are those of the lane coder (the same steps on the same
-// state). There is no lane-dependent branch: every lane runs the same code and stores the same
-// values to the same addresses, so the compiler can never run the wave's lanes apart (with a
-// lane-0-only tail it had sent the other lanes into the next block's loop without lane 0).
-__device__ void mq_code_wave(const MqParams& P, uint32_t cb, uint32_t tabv, int lane) {
-    const T1Info inf = P.info[cb];
-    const uint32_t np = inf.passes;
-    if (np == 0) {
-        P.code_len[cb] = 0;
-        return;
-    }
-    const unsigned long long obase = P.out_off[cb];
-    uint8_t* const out = P.out + obase;
-    uint32_t cap = out_capacity(inf);  // a multiple of 64, as every block's offset
-    bool overflow = obase + cap > P.out_cap;
-    if (overflow) cap = 0;
-    const uint32_t q0 = (uint32_t)__builtin_amdgcn_readlane((int)tabv, 0);
-    const uint32_t q3 = (uint32_t)__builtin_amdgcn_readlane((int)tabv, 3);
-    const uint32_t q4 = (uint32_t)__builtin_amdgcn_readlane((int)tabv, 4);
-    const uint32_t q46 = (uint32_t)__builtin_amdgcn_readlane((int)tabv, 46);
-    uint32_t ctxv = q0;
-    ctxv = lane == 0 ? q4 : ctxv;
-    ctxv = lane == 17 ? q3 : ctxv;
-    ctxv = lane == 18 ? q46 : ctxv;
-    uint32_t A = 0x8000u, C = 0u, B = 0u;
-    int CT = 12, bp = -1;
-    unsigned long long acc = 0ull;  // finished bytes of the current aligned 8-byte group
-    uint32_t flushed = 0;
-    auto byteout = [&]() {
-        const uint32_t carry = B != 0xFFu ? (C >> 27) & 1u : 0u;
-        B += carry;
-        C -= carry << 27;
-        const bool stuff = B == 0xFFu;
-        acc |= (unsigned long long)B << (8 * (bp & 7));
-        if (bp >= 0 && (bp & 7) == 7) {
-            const uint32_t at = (uint32_t)bp & ~7u;
-            if (at < cap) *(unsigned long long*)(out + at) = acc;
-            else overflow = true;
-            acc = 0ull;
-            flushed = at + 8u;
-        }
-        ++bp;
-        B = stuff ? C >> 20 : (C >> 19) & 0xFFu;
-        C &= stuff ? 0xFFFFFu : 0x7FFFFu;
-        CT = stuff ? 7 : 8;
-    };
-    const uint32_t* pend = P.pass_end + (size_t)cb * kMaxPasses;
-    MqSnapshot* snaps = P.snaps + (size_t)cb * kMaxPasses;
-    uint32_t k = 0, pos = 0, next_end = pend[0];
-    const uint2* chunk = P.chunks + (size_t)cb * kMaxPlanes;
-    for (uint32_t j = 0; j < inf.planes; ++j) {
-        const uint2 ch = chunk[j];
-        const uint8_t* src = P.pool + ((unsigned long long)ch.x << 4);
-        for (uint32_t base = 0; base < ch.y; base += 256u) {
-            // 256 symbols at a time, 4 per lane; lanes past the plane's end read its first
-            // word again (a plane's symbols start 64-byte aligned)
-            const uint32_t cnt = ch.y - base < 256u ? ch.y - base : 256u;
-            const uint32_t lo = 4u * (uint32_t)lane < cnt ? 4u * (uint32_t)lane : 0u;
-            const uint32_t wv = *(const uint32_t*)(src + base + lo);
-            for (uint32_t i = 0; i < cnt; ++i) {
-                while (pos == next_end) {  // pass ends: the truncation reference of the pass
-                    snaps[k] = MqSnapshot{bp, B | ((uint32_t)CT << 16), C, A};
-                    ++k;
-                    next_end = k < np ? pend[k] : 0xFFFFFFFFu;
-                }
-                const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)wv, (int)(i >> 2));
-                const uint32_t sv = (word >> (8u * (i & 3u))) & 0xFFu;
-                const uint32_t cx = sv >> 1;
-                const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)ctxv, (int)cx);
-                const uint32_t qe = st & 0xFFFFu;
-                const uint32_t a = A - qe;
-                const bool is_mps = (int)(st ^ (sv << 31)) >= 0;
-                const bool add_c = is_mps != (a < qe);
-                C += add_c ? qe : 0u;
-                A = add_c ? a : qe;
-                if (!is_mps || a < 0x8000u) {
-                    const uint32_t nidx = is_mps ? ((st >> 16) & 63u) : ((st >> 22) & 63u);
-                    const uint32_t msb = is_mps ? st : st ^ (st << 3);
-                    const uint32_t t_new =
-                        (msb & 0x80000000u) | (uint32_t)__builtin_amdgcn_readlane((int)tabv, (int)nidx);
-                    ctxv = lane == (int)cx ? t_new : ctxv;
-                    int nsh = __clz((int)A) - 16;
-                    A <<= nsh;
-                    while (nsh >= CT) {
-                        C <<= CT;
-                        nsh -= CT;
-                        byteout();
-                    }
-                    C <<= nsh;
-                    CT -= nsh;
-                }
-                ++pos;
-            }
-        }
-    }
-    while (pos == next_end) {
-        snaps[k] = MqSnapshot{bp, B | ((uint32_t)CT << 16), C, A};
-        ++k;
-        next_end = k < np ? pend[k] : 0xFFFFFFFFu;
-    }
-    // FLUSH (C.2.9)
-    const uint32_t tempc = C + A;
-    C |= 0xFFFFu;
-    if (C >= tempc) C -= 0x8000u;
-    C <<= CT;
-    byteout();
-    C <<= CT;
-    byteout();
-    uint32_t len = (uint32_t)bp;
-    if (B != 0xFFu) {
-        acc |= (unsigned long long)B << (8 * (bp & 7));
-        len = (uint32_t)bp + 1;
-    }
-    if (len > cap) overflow = true;
-    if (overflow) {
-        atomicOr(&P.counters->flags, 2u);
-        P.code_len[cb] = 0;
-        return;
-    }
-    const uint32_t nw = (len + 3u) >> 2;
-    for (uint32_t wi = flushed >> 2; wi < nw; ++wi)
-        *(uint32_t*)(out + 4u * wi) = (uint32_t)(acc >> (32u * (wi & 1u)));
-    mq_pass_lengths(out, len, snaps, np, P.pass_len + (size_t)cb * kMaxPasses);
-    P.code_len[cb] = len;
-}
-
-// GROUP lanes per workgroup; NQ: 16-byte words of symbols read per lane at a time (1 or 4),
-// with the following NQ in flight while these are coded.
+// One lane per code-block, P.lanes blocks per wave. GROUP lanes per workgroup; NQ: 16-byte
+// groups of symbols read per lane at a time (1 or 4), the following ones in flight while these
+// are coded. A lane goes on to its next plane by itself; the lanes of a wave only share the
+// steps within NQ groups.
+//
+// Large launches are bound by VALU issue: 40 wave-instructions per 64 symbols (35 in the four
+// unrolled steps of a word, the rest bytes taken, pass ends and the cursor), 2.12 ms for 16 4K
+// frames (1,650 M symbols) where a coder that took each byte when it was due spent 94 and
+// 6.1 ms: some lane of 64 had a byte on nearly every step. Small launches are bound by the
+// longest block's chain: about 155 cycles a symbol in the steps (state -> successors from LDS ->
+// state, the interval beside it) and 60-130 in the rest; one 4K frame 1.63 ms (3.0 before), one
+// 512x256 frame 1.23 ms (2.1). What shapes the steps is latency: a dependent VALU operation
+// takes 9 cycles, LDS 50, but a mask that goes through a scalar instruction 20 more and a
+// branch on a vector comparison 28, so there are no scalar mask operations in the steps and
+// one branch per four symbols.
 template <int GROUP, int NQ>
 __global__ void __launch_bounds__(GROUP) t1_mq_kernel(MqParams P) {
-    __shared__ uint32_t s_ctx[19][GROUP];
-    __shared__ uint32_t s_tab[48];
-    if (threadIdx.x < 47) s_tab[threadIdx.x] = kMqTable[threadIdx.x];
+    __shared__ uint32_t s_ctx[kMqContexts][GROUP];
+    __shared__ uint2 s_next[kMqCoderStates];
+    for (int i = threadIdx.x; i < kMqCoderStates; i += GROUP)
+        s_next[i] = make_uint2(kMqTable[2 * i], kMqTable[2 * i + 1]);
     __syncthreads();
     // A full symbol pool left some chunk tables unwritten: nothing to code, the host
     // re-runs Tier-1 with a larger pool.
     if (P.counters->flags & 1u) return;
-    constexpr uint32_t kGroupBytes = 16u * NQ;
     const int t = threadIdx.x;
-    // The nlong longest blocks (the leading entries of the order) one per wave first, by a
-    // fixed stride over the grid's waves (the grid has at least nlong waves when it can).
-    {
-        const int lane = t & 63;
-        const uint32_t tabv = lane < 47 ? s_tab[lane] : 0u;
-        const uint32_t wave =
-            (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (GROUP / 64) + ((uint32_t)t >> 6)));
-        const uint32_t nwaves = gridDim.x * (GROUP / 64);
-        for (uint32_t i = wave; i < P.nlong; i += nwaves) mq_code_wave(P, P.perm[i], tabv, lane);
-    }
-    const uint32_t nrest = P.nblocks - P.nlong;
+    const uint32_t lane = (uint32_t)t & 63u;
+    // Lanes beyond P.lanes code the same blocks again, to the same bytes: a wave of a few active
+    // lanes runs slower than a full one (a dependent VALU operation takes 17-23 cycles instead
+    // of 9 in waves of one active lane, four to a CU).
+    const uint32_t mine = lane % P.lanes;
+    // the lane's context states, GROUP words apart
+    char* const slots = (char*)&s_ctx[0][t];
+    constexpr int kSlotShift = GROUP == 64 ? 8 : (GROUP == 128 ? 9 : 10);
     for (;;) {
-        // one wave-sized group of blocks at a time, in largest-first order
+        // P.lanes blocks at a time, in largest-first order
         uint32_t base = 0;
-        if ((t & 63) == 0) base = atomicAdd(P.work_next, 64u);
+        if (lane == 0) base = atomicAdd(P.work_next, P.lanes);
         base = (uint32_t)__builtin_amdgcn_readfirstlane(__shfl((int)base, 0));
-        if (base >= nrest) break;
-        const uint32_t gid = P.nlong + base + (t & 63);
-        if (gid >= P.nblocks) continue;
-        const uint32_t cb = P.perm[gid];
+        if (base >= P.nblocks) break;
+        const uint32_t cb = P.perm[min(base + mine, P.nblocks - 1u)];
         const T1Info inf = P.info[cb];
         const uint32_t np = inf.passes;
         if (np == 0) {
@@ -932,190 +857,219 @@ __global__ void __launch_bounds__(GROUP) t1_mq_kernel(MqParams P) {
         const unsigned long long obase = P.out_off[cb];
         uint8_t* out = P.out + obase;
         uint32_t cap = out_capacity(inf);  // a multiple of 64, as every block's offset
-        uint32_t overflow = obase + cap > P.out_cap ? 1u : 0u;  // a word, not a lane mask, in the hot loop
-        if (overflow) cap = 0;
-        for (int i = 0; i < 19; ++i) s_ctx[i][t] = s_tab[0];
-        s_ctx[0][t] = s_tab[4];
-        s_ctx[17][t] = s_tab[3];
-        s_ctx[18][t] = s_tab[46];
-        uint32_t A = 0x8000u, C = 0u, B = 0u;
-        int CT = 12, bp = -1;
-        // Finished bytes of the current aligned 8-byte group. The byte at bp = -1 is the
-        // coder's initial dummy: it is 0 and takes no carry (C + A stays within 2^27 until the
-        // first byte-out), so OR-ing it in changes nothing.
-        unsigned long long acc = 0ull;
-        uint32_t flushed = 0;           // codeword bytes already written out (a multiple of 8)
-        // BYTEOUT (C.2.7) with the pending byte B kept in a register: it is final once the
-        // next byte starts. Branch-free but for the 8-byte flush; the wave runs it whenever
-        // one lane needs it, so it is kept short.
-        auto byteout = [&]() {
-            // a carry into B unless B is 0xFF; a B of 0xFF (before or after the carry) is
-            // followed by a stuffed byte of 7 bits
-            const uint32_t carry = B != 0xFFu ? (C >> 27) & 1u : 0u;
-            B += carry;
-            C -= carry << 27;
-            const bool stuff = B == 0xFFu;
-            acc |= (unsigned long long)B << (8 * (bp & 7));
-            if (((uint32_t)bp & 0x80000007u) == 7u) {  // bp >= 0 ends a group
-                const uint32_t at = (uint32_t)bp & ~7u;
-                if (at < cap) *(unsigned long long*)(out + at) = acc;  // cap: a multiple of 64
-                else overflow = 1u;
-                acc = 0ull;
-                flushed = at + 8u;
+        if (obase + cap > P.out_cap) cap = 0;
+        for (int i = 0; i < 19; ++i) s_ctx[i][t] = kMqInitial[0];
+        s_ctx[0][t] = kMqInitial[1];
+        s_ctx[17][t] = kMqInitial[2];
+        s_ctx[18][t] = kMqInitial[3];
+        s_ctx[19][t] = 0;          // neutral symbols: Qe = 0, always the MPS
+        uint32_t A = 0x80000000u;  // A << 16
+        MqCode m{0ull, 12 + 16, 0u, -1};
+        // The bp & 7 finished bytes of the current aligned 8-byte group, the last one lowest. The
+        // byte at bp = -1 is the coder's initial dummy: it is 0 and takes no carry (C + A stays
+        // within 2^27 until the first byte-out), and ends a group that is not written.
+        uint64_t acc = 0ull;
+        // count (1..4) finished bytes, the last one lowest
+        auto put = [&](uint32_t bytes, uint32_t count) {
+            const uint32_t have = ((uint32_t)m.bp & 7u) + count;
+            if (have < 8u) {
+                acc = (acc << (8u * count)) | bytes;
+            } else {
+                const uint32_t over = have - 8u;
+                const uint64_t group = (acc << (8u * (count - over))) | (bytes >> (8u * over));
+                const uint32_t at = (uint32_t)m.bp & ~7u;
+                if (at < cap) *(uint64_t*)(out + at) = __builtin_bswap64(group);  // cap: a multiple of 64
+                acc = bytes & ((1u << (8u * over)) - 1u);
             }
-            ++bp;
-            B = stuff ? C >> 20 : (C >> 19) & 0xFFu;
-            C &= stuff ? 0xFFFFFu : 0x7FFFFu;
-            CT = stuff ? 7 : 8;
+            m.bp += (int)count;
         };
-        const uint32_t* pend = P.pass_end + (size_t)cb * kMaxPasses;
-        MqSnapshot* snaps = P.snaps + (size_t)cb * kMaxPasses;
-        // the next pass end and the one after it: the load of each pass end is issued a
-        // whole pass before the coder reaches it
-        uint32_t k = 0, pos = 0, next_end = pend[0], after_end = np > 1 ? pend[1] : 0xFFFFFFFFu;
+        // BYTEOUT for every byte that is due
+        auto take_bytes = [&]() {
+            if (m.D <= 16) {
+                // all of them at once unless one is 0xFF: the pending byte with its carry and
+                // the due ones but the last, which becomes the pending one
+                const uint32_t k = 16u - (uint32_t)m.D, count = (k >> 3) + 1u, sh = 24u + (k & 7u);
+                const uint64_t V = m.L >> sh;
+                const uint32_t bytes = (m.B << (8u * (count - 1u))) + (uint32_t)(V >> 8);
+                if (m.B != 0xFFu && !((~bytes - 0x01010101u) & bytes & 0x80808080u)) {
+                    put(bytes, count);
+                    m.L -= V << sh;
+                    m.B = (uint32_t)V & 0xFFu;
+                    m.D += (int)(8u * count);
+                } else {
+                    do put(m.byteout(), 1u);
+                    while (m.D <= 16);
+                }
+            }
+        };
+        MqSnapshot* snap = P.snaps + (size_t)cb * kMaxPasses;
         const uint2* chunk = P.chunks + (size_t)cb * kMaxPlanes;
         const uint32_t planes = inf.planes;
-        uint2 ch = chunk[0];
-        // A plane's symbols start 64-byte aligned and take a multiple of 64 bytes of the
-        // pool, so whole groups can be read.
+        // The groups are read two steps ahead: q is being coded, n has arrived (the last symbol
+        // of q looks up the first context of n), the next are in flight. A plane's symbols start
+        // 64-byte aligned and take a multiple of 64 bytes of the pool, so NQ groups can be read
+        // from any multiple of NQ.
+        // No load depends on a condition and what is loaded is next touched a step later, so that
+        // no step waits for memory.
+        const uint2 ch = chunk[0];
         const uint8_t* src = P.pool + ((unsigned long long)ch.x << 4);
-        uint4 q[NQ];
+        uint32_t left = ch.y >> 4;  // 16-byte groups from src to the end of the plane; 0: no more
+        uint32_t j = planes > 1 ? 1u : 0u;
+        uint2 chn = chunk[j];       // the next plane's, if j is one
+        // the groups at src (the pool's first when there are no more), how many of them are the
+        // plane's, and on to the next
+        auto read = [&](uint4(&g)[NQ]) {
 #pragma unroll
-        for (int e = 0; e < NQ; ++e) q[e] = *(const uint4*)(src + 16 * e);
+            for (int e = 0; e < NQ; ++e) g[e] = *(const uint4*)(src + 16 * e);
+            const uint32_t count = left < (uint32_t)NQ ? left : (uint32_t)NQ;
+            const bool more = left > (uint32_t)NQ;
+            const uint8_t* const next = P.pool + ((unsigned long long)chn.x << 4);
+            src = more ? src + 16 * NQ : next;
+            left = more ? left - NQ : (j ? chn.y >> 4 : 0u);
+            j = more ? j : (j && j + 1 < planes ? j + 1 : 0u);
+            chn = chunk[j];
+            return count;
+        };
+        uint4 q[NQ], n[NQ];
+        uint32_t nq = read(q), nn = read(n);
         // the state of the next symbol's context and that context's slot
-        uint32_t* cslot = &s_ctx[(q[0].x & 0xFFu) >> 1][t];
+        uint32_t* cslot = (uint32_t*)(slots + (((q[0].x & 0xFFu) >> 1) << kSlotShift));
         uint32_t t_cur = *cslot;
-        for (uint32_t j = 0; j < planes; ++j) {
-            const uint2 chn = j + 1 < planes ? chunk[j + 1] : make_uint2(0u, 0u);
-            const uint8_t* srcn = P.pool + ((unsigned long long)chn.x << 4);
-            const uint32_t ngroups = (ch.y + kGroupBytes - 1u) / kGroupBytes;
-            if (ngroups == 0 && j + 1 < planes) {  // an empty plane: the next plane's group now
-#pragma unroll
-                for (int e = 0; e < NQ; ++e) q[e] = *(const uint4*)(srcn + 16 * e);
-            }
-            for (uint32_t g = 0; g < ngroups; ++g) {
-                const uint8_t* nsrc = g + 1 < ngroups ? src + kGroupBytes * (g + 1) : (j + 1 < planes ? srcn : nullptr);
-                uint4 n[NQ];
-#pragma unroll
-                for (int e = 0; e < NQ; ++e) n[e] = nsrc ? *(const uint4*)(nsrc + 16 * e) : make_uint4(0u, 0u, 0u, 0u);
-                const uint32_t mg = ch.y - kGroupBytes * g < kGroupBytes ? ch.y - kGroupBytes * g : kGroupBytes;
-                // one copy of the 16 unrolled symbol steps: the group's 16-byte words move
-                // to the front of q in turn
+        for (;;) {
+            uint4 f[NQ];
+            const uint32_t nf = read(f);
 #pragma unroll 1
-                for (int sub = 0; sub < NQ; ++sub) {
-                    if (16u * sub < mg) {
-                        const uint32_t m = mg - 16u * sub < 16u ? mg - 16u * sub : 16u;
-                        // the symbol after this run of m: in the group, or the first of the next
-                        const uint32_t after = 16u * sub + 16u < mg ? (q[NQ > 1 ? 1 : 0].x & 0xFFu) : (n[0].x & 0xFFu);
-                        const uint4 cur = q[0];
-                        const uint32_t w[5] = {cur.x, cur.y, cur.z, cur.w, after};
+            for (uint32_t sub = 0; sub < (uint32_t)NQ; ++sub) {
+                if (sub < nq) {
+                    uint32_t w = q[0].x, w1 = q[0].y, w2 = q[0].z, w3 = q[0].w;
+                    const uint32_t w4 = NQ > 1 && sub + 1 < nq ? q[NQ > 1 ? 1 : 0].x : (nn ? n[0].x : 0u);
 #pragma unroll
-                        for (uint32_t b = 0; b < 16; ++b) {
-                            if (b < m) {  // a guard, not an exit, so the 16 steps unroll
-                                // pass ends: the coder state is the truncation reference of the pass
-                                while (pos == next_end) {
-                                    snaps[k] = MqSnapshot{bp, B | ((uint32_t)CT << 16), C, A};
-                                    ++k;
-                                    next_end = after_end;
-                                    after_end = k + 1 < np ? pend[k + 1] : 0xFFFFFFFFu;
-                                }
-                                const uint32_t sv = (w[b >> 2] >> (8 * (b & 3))) & 0xFFu;
-                                const uint32_t sn = b + 1 < m ? (w[(b + 1) >> 2] >> (8 * ((b + 1) & 3))) & 0xFFu : w[4];
-                                // the next symbol's context state, read before this symbol may change it
-                                uint32_t* const nslot = &s_ctx[sn >> 1][t];
-                                const uint32_t t_next = *nslot;
-                                const uint32_t st = t_cur;
-                                const uint32_t qe = st & 0xFFFFu;
-                                const uint32_t a = A - qe;  // A <= 0xFFFF, so a < 0x10000
-                                const bool is_mps = (int)(st ^ (sv << 31)) >= 0;  // the decision equals the MPS
-                                const bool add_c = is_mps != (a < qe);  // conditional exchange (C.2.5 / C.2.6)
-                                C += add_c ? qe : 0u;
-                                A = add_c ? a : qe;
-                                // The state changes and A, C renormalise unless the symbol is
-                                // the MPS with A still >= 0x8000; then the shift count below is
-                                // 0 and the state written back is the old one, so every lane
-                                // runs the same instructions and only byte-out branches. After
-                                // an LPS the MPS flips where SWITCH (bit 28) is set.
-                                const bool renorm = !is_mps || a < 0x8000u;
-                                const uint32_t nidx = is_mps ? ((st >> 16) & 63u) : ((st >> 22) & 63u);
-                                const uint32_t msb = is_mps ? st : st ^ (st << 3);
-                                const uint32_t t_new = (msb & 0x80000000u) | s_tab[nidx];
-                                const uint32_t st_new = renorm ? t_new : st;
-                                *cslot = st_new;
-                                // RENORME: A and C shift until A >= 0x8000 (at most 15 bits), a
-                                // byte out whenever CT runs out; a second one is rare (an LPS
-                                // with a small Qe). A is never 0 here.
-                                int nsh = __builtin_clz(A) - 16;
-                                A <<= nsh;
-                                int sh = nsh < CT ? nsh : CT;
-                                C <<= sh;
-                                CT -= sh;
-                                if (CT == 0) {
-                                    nsh -= sh;
-                                    do {
-                                        byteout();
-                                        sh = nsh < CT ? nsh : CT;
-                                        C <<= sh;
-                                        CT -= sh;
-                                        nsh -= sh;
-                                    } while (CT == 0);
-                                }
-                                t_cur = nslot == cslot ? st_new : t_next;
-                                cslot = nslot;
-                                ++pos;
-                            }
+                    for (int k = 0; k < 4; ++k) {
+                        // Four symbols with the code register assumed to hold them: no byte is
+                        // taken, and what would have needed it is looked at after them.
+                        const uint64_t L0 = m.L;
+                        const int32_t D0 = m.D;
+                        uint32_t adds[4], shifts[4], carries = 0;
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) {
+                            // the next symbol's context state, read before this symbol may change it
+                            const uint32_t nctx = b < 3 ? (w >> (8 * b + 9)) & 31u : (w1 >> 1) & 31u;
+                            uint32_t* const nslot = (uint32_t*)(slots + (nctx << kSlotShift));
+                            const uint32_t t_next = *nslot;
+                            const uint32_t st = t_cur;
+                            const uint2 succ = *(const uint2*)((const char*)s_next + (st & 0x3F8u));
+                            const bool lps = (int)(st ^ (w << (31 - 8 * b))) < 0;
+                            // C.2.5 / C.2.6 with the conditional exchange: the MPS takes the
+                            // larger of a and Qe, the LPS the smaller; C grows by Qe where a,
+                            // the upper part, is taken (on a tie: by the MPS)
+                            const uint32_t qe = st & 0x7FFF0000u;
+                            const uint32_t a = A - qe;
+                            const uint32_t hi = a > qe ? a : qe, lo = a < qe ? a : qe;
+                            const uint32_t below = a < qe ? qe : 0u;
+                            const uint32_t add = (lps ? below : qe - below) >> 11;
+                            A = lps ? lo : hi;
+                            // The state changes and A, C renormalise unless the symbol is the
+                            // MPS with A still >= 0x8000; then the shift count is 0 and the
+                            // state written back is the old one, so every lane runs the same
+                            // instructions.
+                            const uint32_t t_new = lps ? succ.y : succ.x;
+                            const uint32_t st_new = (int)A < 0 ? st : t_new;
+                            *cslot = st_new;
+                            const uint32_t nsh = (uint32_t)__builtin_clz(A);  // A is never 0
+                            A <<= nsh;
+                            uint32_t low;
+                            carries += __builtin_add_overflow((uint32_t)m.L, add, &low) ? 1u : 0u;
+                            m.L = ((m.L & 0xFFFFFFFF00000000ull) | low) << nsh;
+                            m.D -= (int)nsh;
+                            adds[b] = add;
+                            shifts[b] = nsh;
+                            t_cur = nslot == cslot ? st_new : t_next;
+                            cslot = nslot;
                         }
+                        // a pass ends with the word (its top bit), or the register wants looking at
+                        if (__builtin_amdgcn_ballot_w64((m.D | (int32_t)w | (int32_t)(0u - carries)) < 0)) {
+                            asm volatile("");
+                            if (__builtin_amdgcn_ballot_w64((m.D | (int32_t)(0u - carries)) < 0)) {
+                                // The bytes due, of all lanes, so that they are due at the same
+                                // time again. After a carry out of bit 31 (about 1 addition in
+                                // 4,000) or more shifts than the register holds, the symbols'
+                                // additions and shifts once more with the bytes taken in between.
+                                int r = 4;
+                                if (__builtin_amdgcn_ballot_w64(carries != 0u || m.D < -15)) {
+                                    m.L = L0;
+                                    m.D = D0;
+                                    r = 0;
+                                }
+                                for (;; ++r) {
+                                    take_bytes();
+                                    if (r == 4) break;
+                                    m.L = (m.L + adds[0]) << shifts[0];
+                                    m.D -= (int)shifts[0];
+                                    adds[0] = adds[1], adds[1] = adds[2], adds[2] = adds[3];
+                                    shifts[0] = shifts[1], shifts[1] = shifts[2], shifts[2] = shifts[3];
+                                }
+                            }
+                            if ((int32_t)w < 0)  // the coder state is the truncation reference of the pass
+                                *snap++ = MqSnapshot{((uint32_t)(m.bp + 1) << 16) | (m.B << 8) | (uint32_t)m.D,
+                                                     (uint32_t)m.L, (uint32_t)(m.L >> 32), A};
+                        }
+                        w = w1;
+                        w1 = w2;
+                        w2 = w3;
+                        w3 = w4;
                     }
-#pragma unroll
-                    for (int e = 0; e + 1 < NQ; ++e) q[e] = q[e + 1];
                 }
 #pragma unroll
-                for (int e = 0; e < NQ; ++e) q[e] = n[e];
+                for (int e = 0; e + 1 < NQ; ++e) q[e] = q[e + 1];
             }
-            ch = chn;
-            src = srcn;
-        }
-        while (pos == next_end) {
-            snaps[k] = MqSnapshot{bp, B | ((uint32_t)CT << 16), C, A};
-            ++k;
-            next_end = after_end;
-            after_end = k + 1 < np ? pend[k + 1] : 0xFFFFFFFFu;
+            if (!nn) break;
+#pragma unroll
+            for (int e = 0; e < NQ; ++e) q[e] = n[e], n[e] = f[e];
+            nq = nn;
+            nn = nf;
         }
         // FLUSH (C.2.9)
-        const uint32_t tempc = C + A;
-        C |= 0xFFFFu;
-        if (C >= tempc) C -= 0x8000u;
-        C <<= CT;
-        byteout();
-        C <<= CT;
-        byteout();
-        uint32_t len = (uint32_t)bp;
-        if (B != 0xFFu) {
-            acc |= (unsigned long long)B << (8 * (bp & 7));
-            len = (uint32_t)bp + 1;
+        take_bytes();
+        {
+            uint32_t C = (uint32_t)(m.L >> 5);
+            const uint32_t tempc = C + (A >> 16);
+            C |= 0xFFFFu;
+            if (C >= tempc) C -= 0x8000u;
+            m.L = (uint64_t)C << 5;
         }
-        // the bytes after the last full group, as whole words
+#pragma unroll 1
+        for (int k = 0; k < 2; ++k) {
+            m.L <<= m.D - 16;
+            m.D = 16;
+            take_bytes();
+        }
+        const uint32_t flushed = (uint32_t)m.bp & ~7u;  // codeword bytes already written out
+        uint32_t len = (uint32_t)m.bp, have = len & 7u;
+        if (m.B != 0xFFu) {
+            acc = (acc << 8) | m.B;
+            ++len;
+            ++have;
+        }
+        acc = have ? __builtin_bswap64(acc << (8u * (8u - have))) : 0ull;
         if (len > cap) {
-            overflow = 1u;
-        } else {
-            const uint32_t nw = (len + 3u) >> 2;
-            for (uint32_t wi = flushed >> 2; wi < nw; ++wi)
-                *(uint32_t*)(out + 4u * wi) = (uint32_t)(acc >> (32u * (wi & 1u)));
-        }
-        if (overflow) {
             atomicOr(&P.counters->flags, 2u);
             P.code_len[cb] = 0;
             continue;
         }
-        mq_pass_lengths(out, len, snaps, np, P.pass_len + (size_t)cb * kMaxPasses);
+        // the bytes after the last full group, as whole words
+        const uint32_t nw = (len + 3u) >> 2;
+        for (uint32_t wi = flushed >> 2; wi < nw; ++wi)
+            *(uint32_t*)(out + 4u * wi) = (uint32_t)(acc >> (32u * (wi & 1u)));
+        mq_pass_lengths(out, len, cap, P.snaps + (size_t)cb * kMaxPasses, np, P.pass_len + (size_t)cb * kMaxPasses);
         P.code_len[cb] = len;
     }
 }
 
 static hipError_t upload_mq_table() {
-    uint32_t tab[47];
-    build_mq_table(tab);
-    return hipMemcpyToSymbol(HIP_SYMBOL(kMqTable), tab, sizeof tab);
+    uint32_t tab[2 * kMqCoderStates], initial[4];
+    build_mq_coder_table(tab, initial);
+    const hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(kMqTable), tab, sizeof tab);
+    return e != hipSuccess ? e : hipMemcpyToSymbol(HIP_SYMBOL(kMqInitial), initial, sizeof initial);
 }
 
 hipError_t t1_tables_init() { return upload_mq_table(); }

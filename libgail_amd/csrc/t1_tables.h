@@ -54,4 +54,23 @@ inline void build_mq_table(uint32_t tab[47]) {
         tab[i] = qe[i] | ((uint32_t)nm[i] << 16) | ((uint32_t)nl[i] << 22) | ((i == 0 || i == 6 || i == 14) ? 1u << 28 : 0u);
 }
 
+// The MQ encoder's states: state 2 * i + m is row i of Table C.2 with MPS m, as the word
+// MPS << 31 | Qe << 16 | state * 8, the last the byte offset of the state's successors in tab:
+// tab[2 * state] after an MPS, tab[2 * state + 1] after an LPS (the MPS flipped where SWITCH
+// says so). initial: the words of rows 0, 4, 3 and 46 with MPS 0, where contexts start
+// (Table D.7).
+constexpr int kMqCoderStates = 94;
+inline void build_mq_coder_table(uint32_t tab[2 * kMqCoderStates], uint32_t initial[4]) {
+    uint32_t t[47];
+    build_mq_table(t);
+    auto word = [&](uint32_t i, uint32_t m) { return (m << 31) | ((t[i] & 0xFFFFu) << 16) | ((2 * i + m) * 8); };
+    for (uint32_t i = 0; i < 47; ++i)
+        for (uint32_t m = 0; m < 2; ++m) {
+            tab[2 * (2 * i + m)] = word((t[i] >> 16) & 63u, m);
+            tab[2 * (2 * i + m) + 1] = word((t[i] >> 22) & 63u, m ^ ((t[i] >> 28) & 1u));
+        }
+    const uint32_t rows[4] = {0, 4, 3, 46};
+    for (int k = 0; k < 4; ++k) initial[k] = word(rows[k], 0);
+}
+
 }  // namespace gail_amd
