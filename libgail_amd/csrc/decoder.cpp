@@ -15,7 +15,7 @@ namespace gail_amd {
 
 namespace {
 
-// Bytes a lane may read past a codeword's end (the 16-byte window, aligned down to 8).
+// Bytes a wave may read past a codeword's end (less than a dword of its window).
 constexpr size_t kBytePad = 64;
 // Length classes of the block ordering (bytes / 4, longer blocks share the top class).
 constexpr uint32_t kLenKeys = 4096;
@@ -57,7 +57,7 @@ Decoder::Decoder(int device, const Layout& L, int reduce, bool highBits)
     if (reduce < 0 || reduce > L.levels) throw std::runtime_error("more resolution levels left out than the stream has");
     try {
         hipCheck(hipSetDevice(dev_), "hipSetDevice");
-        cus_ = DeviceContext::get(dev_).computeUnits();
+        DeviceContext::get(dev_);  // the kernels' tables
         ws_.resize(L_.levels + 1);
         hs_.resize(L_.levels + 1);
         ws_[0] = L_.width;
@@ -80,7 +80,7 @@ Decoder::Decoder(int device, const Layout& L, int reduce, bool highBits)
         hipCheck(hipMalloc(&dOut_, outBytes), "decoder picture");
         hipCheck(hipHostMalloc((void**)&hOut_, outBytes, hipHostMallocDefault), "decoder picture (pinned)");
         ensureBytes(1500000);  // a DCI frame is at most 250 Mbit/s over 24 frames
-        ensureDescs(((size_t)wanted_.size() / kDecSlots + 1) * kDecSlots);
+        ensureDescs(wanted_.size());
     } catch (...) {
         release();
         throw;
@@ -135,37 +135,24 @@ void Decoder::ensureDescs(size_t n) {
     capDescs_ = cap;
 }
 
-void DescPlan::plan(const Layout& L, const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks,
-                    int cus) {
+void DescPlan::plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks) {
     // Coded blocks longest first (a counting sort over length classes).
     count.assign(kLenKeys + 1, 0u);
-    uint64_t total = 0;
     size_t ncoded = 0;
     auto key = [](uint32_t len) { return kLenKeys - 1u - std::min(len >> 2, kLenKeys - 1u); };
     for (size_t k = 0; k < wanted.size(); ++k)
         if (coded[k]) {
             ++count[key(blocks[wanted[k]].len) + 1];
-            total += blocks[wanted[k]].len;
             ++ncoded;
         }
     for (uint32_t k = 0; k < kLenKeys; ++k) count[k + 1] += count[k];
     order.resize(ncoded);
     for (size_t k = 0; k < wanted.size(); ++k)
         if (coded[k]) order[count[key(blocks[wanted[k]].len)]++] = (uint32_t)wanted[k];
-    // Waves: a wave runs as long as its longest lane, so a long block takes a wave of its own
-    // and short ones share, up to kDecWaveLanes blocks and a byte budget that spreads the frame
-    // over about eight waves per compute unit (measured best on 4K frames at 250 Mbit/s).
-    budget = std::max<uint64_t>(384, total / (uint64_t)(8 * cus));
-    // blocks over the budget would sit alone in a wave: they get a whole wave each and are
-    // decoded with the wave's scalar unit
-    nlong = 0;
-    while (nlong < order.size() && blocks[order[nlong]].len > budget) ++nlong;
-    (void)L;
 }
 
-uint32_t DescPlan::pack(const Layout& L, const DecCode* blocks, DecBlock* out) const {
-    const uint32_t lanes = (uint32_t)kDecWaveLanes;
-    auto entry = [&](uint32_t i) {
+void DescPlan::pack(const Layout& L, const DecCode* blocks, DecBlock* out) const {
+    for (const uint32_t i : order) {
         const DecCode& c = blocks[i];
         const CodeBlock& cb = L.cblks[i];
         const Subband& b = L.bands[cb.band];
@@ -176,49 +163,15 @@ uint32_t DescPlan::pack(const Layout& L, const DecCode* blocks, DecBlock* out) c
                  ((uint32_t)c.nbps << 12) | ((uint32_t)c.passes << 18);
         d.dst = (uint32_t)b.comp * (uint32_t)L.width * (uint32_t)L.height +
                 (uint32_t)(b.py0 + cb.y0) * (uint32_t)L.width + (uint32_t)(b.px0 + cb.x0);
-        return d;
-    };
-    uint32_t n = 0, inWave = 0;
-    uint64_t waveBytes = 0;
-    for (uint32_t k = 0; k < nlong; ++k, ++n)
-        if (out) out[n] = entry(order[k]);
-    for (uint32_t k = nlong; k < order.size(); ++k) {
-        const uint32_t i = order[k];
-        const DecCode& c = blocks[i];
-        if (inWave && (inWave == lanes || waveBytes + c.len > budget)) {
-            if (out)
-                for (; inWave < lanes; ++inWave) out[n++] = DecBlock{0, 0, 0, kDecEmpty};
-            else
-                n += lanes - inWave;
-            inWave = 0;
-            waveBytes = 0;
-        }
-        if (out) out[n] = entry(i);
-        ++n;
-        ++inWave;
-        waveBytes += c.len;
+        *out++ = d;
     }
-    if (inWave) {
-        if (out)
-            for (; inWave < lanes; ++inWave) out[n++] = DecBlock{0, 0, 0, kDecEmpty};
-        else
-            n += lanes - inWave;
-    }
-    // whole workgroups
-    while (t1_decode_waves(n, nlong) % (uint32_t)kDecWaves) {
-        for (uint32_t j = 0; j < lanes; ++j, ++n)
-            if (out) out[n] = DecBlock{0, 0, 0, kDecEmpty};
-    }
-    return n;
 }
 
 uint32_t Decoder::buildDescs(const uint8_t* coded, const DecCode* blocks) {
-    plan_.plan(L_, wanted_, coded, blocks, cus_);
-    const uint32_t n = plan_.pack(L_, blocks, nullptr);
-    ensureDescs(n);
+    plan_.plan(wanted_, coded, blocks);
+    ensureDescs(plan_.order.size());
     plan_.pack(L_, blocks, hDescs_);
-    nlong_ = plan_.nlong;
-    return n;
+    return (uint32_t)plan_.order.size();
 }
 
 void queueDecode(const Layout& L, const Layout& frame, int reduce, bool highBits, const DecodeBuffers& b, hipStream_t s,
@@ -229,7 +182,6 @@ void queueDecode(const Layout& L, const Layout& frame, int reduce, bool highBits
     tp.bytes = b.bytes;
     tp.blocks = b.descs;
     tp.nblocks = b.nd;
-    tp.nlong = b.nlong;
     tp.words = b.words;
     tp.nwords = (uint32_t)(3 * npix);
     tp.stride = W;
@@ -346,7 +298,6 @@ void Decoder::decode(const Layout& frame, const uint8_t* data, size_t size, cons
     buf.bytes = dBytes_;
     buf.descs = dDescs_;
     buf.nd = nd;
-    buf.nlong = nlong_;
     buf.words = dWords_;
     buf.plane[0] = dPlane_[0];
     buf.plane[1] = dPlane_[1];
@@ -394,8 +345,8 @@ namespace {
 
 // Intermediate buffers of one frame of up to kNoAllocMaxWidth x kNoAllocMaxHeight: the
 // reconstruction words and the two float plane sets (3 x 2048 x 1080 x 4 bytes each), the
-// codestream with its read-ahead pad, and the Tier-1 table (up to 16 entries per block when
-// every wave holds one block, for the 6,708 blocks of a 2K frame).
+// codestream with its read-ahead pad, and the Tier-1 table (16 bytes for each of the 6,708
+// blocks of a 2K frame).
 constexpr size_t kNoAllocPlane = (size_t)3 * kNoAllocMaxWidth * kNoAllocMaxHeight * 4;
 constexpr size_t kNoAllocCodeBytes = (kNoAllocMaxBytes + kBytePad + 255) / 256 * 256;
 constexpr size_t kNoAllocTableBytes = 2u << 20;
@@ -411,7 +362,6 @@ struct NoAllocDevice {
     std::once_flag once;
     hipError_t setup = hipSuccess;
     uint8_t* base = nullptr;  // scratch's address on this device
-    int cus = 256;
     std::mutex m;             // one call at a time on the shared array
 };
 NoAllocDevice g_noAlloc[kNoAllocDevices];
@@ -424,10 +374,6 @@ void noAllocSetup(NoAllocDevice& d, int device) {
         d.setup = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (d.setup == hipSuccess) d.base = static_cast<uint8_t*>(p);
         if (d.setup == hipSuccess) d.setup = dec_tables_init();
-        int cus = 0;
-        if (d.setup == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-            cus > 0)
-            d.cus = cus;
     });
     hipCheck(d.setup, "no-allocation decoder set-up");
 }
@@ -474,8 +420,8 @@ void decodeNoAlloc(int device, const Layout& frame, int reduce, bool highBits, c
             wanted.push_back(i);
             coded.push_back(c.passes && c.nbps >= 1 && c.nbps <= 30 && (size_t)c.offset + c.len <= size);
         }
-    plan.plan(frame, wanted, coded.data(), blocks, d.cus);
-    const uint32_t nd = plan.pack(frame, blocks, nullptr);
+    plan.plan(wanted, coded.data(), blocks);
+    const uint32_t nd = (uint32_t)plan.order.size();
     if ((size_t)nd * sizeof(DecBlock) > kNoAllocTableBytes) throw std::runtime_error("Tier-1 table larger than its room");
     table.resize(nd);
     plan.pack(frame, blocks, table.data());
@@ -491,7 +437,6 @@ void decodeNoAlloc(int device, const Layout& frame, int reduce, bool highBits, c
     b.bytes = bytes;
     b.descs = descs;
     b.nd = nd;
-    b.nlong = plan.nlong;
     b.out = static_cast<uint8_t*>(dst);
     b.pitch = (int64_t)strideBytes;
 

@@ -26,24 +26,21 @@ struct DecodeTimes {
 
 constexpr int kMaxDecLevels = 8;
 
-// The Tier-1 decode table of one frame: the blocks to decode, longest first; the longest get
-// a wave each, the rest are packed into waves of up to kDecWaveLanes blocks by a byte budget
-// (a wave runs as long as its longest lane).
+// The Tier-1 decode table of one frame: the blocks to decode, a wave each, longest first (they
+// start first, and a frame takes as long as its longest block).
 struct DescPlan {
     std::vector<uint32_t> order, count;
-    uint32_t nlong = 0;
-    uint64_t budget = 0;
     // wanted: the layout's blocks of the resolutions kept; coded[k]: wanted[k] has data.
-    void plan(const Layout& L, const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks, int cus);
-    // Writes the table to out (nullptr: only counts); returns its entries (whole workgroups).
-    uint32_t pack(const Layout& L, const DecCode* blocks, DecBlock* out) const;
+    void plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks);
+    // Writes the table, order.size() entries, to out.
+    void pack(const Layout& L, const DecCode* blocks, DecBlock* out) const;
 };
 
 // Device buffers of one frame's decode.
 struct DecodeBuffers {
     const uint8_t* bytes = nullptr;   // codestream, readable 64 bytes past its end
-    const DecBlock* descs = nullptr;  // nd table entries, the first nlong a wave each
-    uint32_t nd = 0, nlong = 0;
+    const DecBlock* descs = nullptr;  // nd table entries
+    uint32_t nd = 0;
     uint32_t* words = nullptr;        // 3 W x H reconstruction words, zero beforehand
     float* plane[2] = {nullptr, nullptr};  // 3 W x H floats each, the inverse DWT's ping-pong
     float* wave = nullptr;            // dequantised planes wanted (3 W x H floats), or null
@@ -98,8 +95,8 @@ private:
     void release();
     void ensureBytes(size_t n);
     void ensureDescs(size_t n);
-    // Orders the blocks marked in coded[] (one flag per wanted block) longest first, gives the
-    // longest a wave each and packs the rest into waves; returns the table's entries.
+    // Writes the table of the blocks marked in coded[] (one flag per wanted block), longest
+    // first; returns its entries.
     uint32_t buildDescs(const uint8_t* coded, const DecCode* blocks);
 
     int dev_;
@@ -122,8 +119,6 @@ private:
     DecBlock* dDescs_ = nullptr;
     DecBlock* hDescs_ = nullptr;
     size_t capDescs_ = 0;
-    uint32_t nlong_ = 0;  // leading table entries decoded a whole wave each
-    int cus_ = 256;
     std::vector<float> hWave_;
 };
 

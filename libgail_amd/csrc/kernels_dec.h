@@ -7,25 +7,18 @@
 
 namespace gail_amd {
 
-// One lane's code-block. Lanes left empty have dst == kDecEmpty.
+// One code-block to decode.
 struct DecBlock {
     uint32_t off, len;  // the codeword within the codestream buffer
     uint32_t geom;      // (w - 1) | (h - 1) << 5 | orient << 10 | nbps << 12 | passes << 18
     uint32_t dst;       // word index of the block's top-left sample in the Mallat planes
 };
-constexpr uint32_t kDecEmpty = 0xFFFFFFFFu;
-// Only the first kDecWaveLanes lanes of a wave decode blocks (waves are sparse anyway: a wave
-// runs as long as its longest lane, so long blocks go nearly alone), which lets a workgroup
-// of kDecWaves waves keep every decoding lane's state in the LDS a full wave would take.
-constexpr int kDecWaveLanes = 16;
-constexpr int kDecWaves = 4;
-constexpr int kDecSlots = kDecWaveLanes * kDecWaves;
+constexpr int kDecWaves = 4;  // waves, a block each, per workgroup
 
 struct T1DecodeParams {
     const uint8_t* bytes;  // codestream, readable 64 bytes past its end
-    const DecBlock* blocks;  // nlong long blocks (one wave each), then kDecWaveLanes per wave
-    uint32_t nblocks;      // entries, covering whole workgroups of kDecWaves waves
-    uint32_t nlong;
+    const DecBlock* blocks;
+    uint32_t nblocks;
     uint32_t* words;       // 3 Mallat planes of reconstruction words, zero beforehand
     uint32_t nwords;
     uint32_t stride;       // words per plane row (the frame width)
@@ -61,10 +54,6 @@ struct IctPack {
 };
 
 hipError_t dec_tables_init();
-// Waves (and so workgroups) the table of p covers.
-inline uint32_t t1_decode_waves(uint32_t nblocks, uint32_t nlong) {
-    return nlong + (nblocks - nlong) / (uint32_t)kDecWaveLanes;
-}
 hipError_t launch_t1_decode(const T1DecodeParams& p, hipStream_t s);
 void idwt_tile_size(int& tx, int& ty);
 hipError_t launch_idwt_level(const IdwtLevel& p, hipStream_t s);

@@ -1067,7 +1067,7 @@ __global__ void __launch_bounds__(GROUP) t1_mq_kernel(MqParams P) {
 
 static hipError_t upload_mq_table() {
     uint32_t tab[2 * kMqCoderStates], initial[4];
-    build_mq_coder_table(tab, initial);
+    build_mq_coder_table(tab, initial, 16);
     const hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(kMqTable), tab, sizeof tab);
     return e != hipSuccess ? e : hipMemcpyToSymbol(HIP_SYMBOL(kMqInitial), initial, sizeof initial);
 }

@@ -1,6 +1,6 @@
 // EBCOT Tier-1 decoding of one code-block (ISO/IEC 15444-1 Annexes C.3 and D, no mode
-// switches), written once for the GPU kernel (one lane per block) and for a host build
-// that checks it against the CPU decoder.
+// switches), decision by decision in the standard's order: the sequential form of what a wave
+// does in t1_decode_wave.h, for a host build that checks it against the CPU decoder.
 //
 // The block's state is four sets of 32 row masks (bit x = column x): significant, negative,
 // coded in this plane's significance pass, refined before. A stripe's six significance rows

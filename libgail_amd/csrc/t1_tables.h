@@ -54,16 +54,18 @@ inline void build_mq_table(uint32_t tab[47]) {
         tab[i] = qe[i] | ((uint32_t)nm[i] << 16) | ((uint32_t)nl[i] << 22) | ((i == 0 || i == 6 || i == 14) ? 1u << 28 : 0u);
 }
 
-// The MQ encoder's states: state 2 * i + m is row i of Table C.2 with MPS m, as the word
-// MPS << 31 | Qe << 16 | state * 8, the last the byte offset of the state's successors in tab:
-// tab[2 * state] after an MPS, tab[2 * state + 1] after an LPS (the MPS flipped where SWITCH
-// says so). initial: the words of rows 0, 4, 3 and 46 with MPS 0, where contexts start
-// (Table D.7).
+// The MQ coders' states: state 2 * i + m is row i of Table C.2 with MPS m, as the word MPS << 31 |
+// Qe << qe_shift | state * 8, the last the byte offset of the state's successors in tab: tab[2 *
+// state] after an MPS, tab[2 * state + 1] after an LPS (the MPS flipped where SWITCH says so).
+// initial: the words of rows 0, 4, 3 and 46 with MPS 0, where contexts start (Table D.7). The
+// encoder compares unsigned (qe_shift 16), the decoder by sign (15).
 constexpr int kMqCoderStates = 94;
-inline void build_mq_coder_table(uint32_t tab[2 * kMqCoderStates], uint32_t initial[4]) {
+inline void build_mq_coder_table(uint32_t tab[2 * kMqCoderStates], uint32_t initial[4], int qe_shift) {
     uint32_t t[47];
     build_mq_table(t);
-    auto word = [&](uint32_t i, uint32_t m) { return (m << 31) | ((t[i] & 0xFFFFu) << 16) | ((2 * i + m) * 8); };
+    auto word = [&](uint32_t i, uint32_t m) {
+        return (m << 31) | ((t[i] & 0xFFFFu) << qe_shift) | ((2 * i + m) * 8);
+    };
     for (uint32_t i = 0; i < 47; ++i)
         for (uint32_t m = 0; m < 2; ++m) {
             tab[2 * (2 * i + m)] = word((t[i] >> 16) & 63u, m);
@@ -71,6 +73,19 @@ inline void build_mq_coder_table(uint32_t tab[2 * kMqCoderStates], uint32_t init
         }
     const uint32_t rows[4] = {0, 4, 3, 46};
     for (int k = 0; k < 4; ++k) initial[k] = word(rows[k], 0);
+}
+
+// Sign coding (Table D.3) by the left, right, upper and lower neighbour's two bits each
+// (significant | negative << 1, the left one lowest): (context + 1) << 1 | flip.
+inline void build_sign_table(uint8_t t[256]) {
+    for (int i = 0; i < 256; ++i) {
+        auto v = [&](int k) { return ((i >> (2 * k)) & 1) ? (((i >> (2 * k + 1)) & 1) ? -1 : 1) : 0; };
+        int h = std::max(-1, std::min(1, v(0) + v(1))), u = std::max(-1, std::min(1, v(2) + v(3)));
+        const int flip = h < 0 || (h == 0 && u < 0) ? 1 : 0;
+        if (flip) h = -h, u = -u;
+        const int cx = h ? 12 + u : (u ? 10 : 9);
+        t[i] = (uint8_t)((cx + 1) << 1 | flip);
+    }
 }
 
 }  // namespace gail_amd
