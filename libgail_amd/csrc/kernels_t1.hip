@@ -7,10 +7,10 @@
 // right neighbours come from lane shuffles, above and below are bit shifts. Per 4-row
 // stripe the significance-propagation pass is solved as a monotone fixpoint over the
 // half-wave (no change anywhere => the sequential scan's result), cleanup needs no
-// fixpoint because every remaining sample is coded. Each lane packs its column's
-// symbols of a stripe (at most 10, 6 bits each) in a 64-bit register; ballots + mbcnt
-// give the exclusive prefix over the columns, so symbols land in scan order in a per-block
-// LDS staging buffer, copied to an HBM pool once per bit-plane.
+// fixpoint because every remaining sample is coded. Each lane holds its column's symbols of
+// a stripe (at most 10) as bytes of registers; a scan over the half-wave gives the exclusive
+// prefix over the columns, so symbols land in scan order in a per-block LDS staging buffer,
+// copied to an HBM pool once per bit-plane.
 //
 // MQ coding: one lane per code-block, blocks ordered largest first so a wave's lanes
 // finish together. The coder keeps A, C, CT and the pending byte in registers, with several
@@ -93,6 +93,21 @@ __device__ __forceinline__ uint32_t stripe_bytes(uint32_t m, int r0) {
     return t;
 }
 
+// The same at bit J of each byte (J <= 2, so that the multiplier keeps its 24 bits), into w.
+__device__ __forceinline__ uint32_t stripe_bits(uint32_t w, uint32_t m, int r0, int j) {
+    uint32_t t = __umul24((m >> r0) & 0xFu, 0x204081u << j);
+    asm("" : "+v"(t));
+    const uint32_t at = 0x01010101u << j;
+    return (t & at) | (w & ~at);
+}
+
+// The first n (at most 4) bytes of w to out; every lane stores all four, those it does not have
+// to junk, so that no lane diverges.
+__device__ __forceinline__ void put_bytes(uint32_t w, uint32_t n, uint8_t* out, uint8_t* junk) {
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) (j < n ? out : junk)[j] = (uint8_t)(w >> (8 * j));
+}
+
 constexpr int kChunkBytes = 65536;  // symbol pool grabbed per wave at a time
 
 }  // namespace
@@ -139,11 +154,35 @@ hipError_t launch_quant_debug(const T1Block* blocks, const T1Band* bands, const 
 }
 
 // ---------------------------------------------------------------- context modelling
+// Bound by vector issue: 0.86 vector instructions a cycle and CU at 16 4K frames, three waves
+// a SIMD (the magnitudes and planes of a column need 168 registers), LDS busy 40 % of the time
+// with the symbols' byte stores. So instructions are what is saved: the quantiser and the
+// stores have no branches (a lane without a symbol stores to a junk byte), a symbol's bits are
+// set for four rows by one multiplication each, and a stripe's bytes are put in order by
+// v_perm with selectors from a table of all 256 cases. With divergent stores, selectors
+// built per stripe and a masked quantiser the same 16 frames took 5.42 ms (20 % more vector and
+// 57 % more scalar instructions), now 4.80; one 2K frame 0.232 and 0.213, 512x256 0.097 and 0.081.
 template <int WAVES>
 __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
     // a plane's symbols per block, then 128 bytes where each lane writes the symbols its rows
     // do not have (so that every lane stores on every step)
-    __shared__ __attribute__((aligned(16))) uint8_t s_sym[WAVES][2][kPlaneStage + 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_sym[WAVES][2][kPlaneStage + 144];
+    // For the sets of a stripe's rows that have a zero-coding (low nibble) and a sign symbol (high
+    // nibble), the order of their bytes as selectors: the rows in turn, each one's zero-coding
+    // byte (0-3) before its sign byte (4-7).
+    __shared__ uint2 s_order[256];
+    for (uint32_t i = threadIdx.x; i < 256u; i += WAVES * 64) {
+        unsigned long long v = 0x0C0C0C0C0C0C0C0Cull;
+        uint32_t j = 0;
+        for (uint32_t k = 0; k < 8; ++k)
+            if ((i >> (k >> 1 | (k & 1u) << 2)) & 1u) {
+                const uint32_t sel = k >> 1 | (k & 1u) << 2;
+                v = (v & ~(0xFFull << (8 * j))) | ((unsigned long long)sel << (8 * j));
+                ++j;
+            }
+        s_order[i] = make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+    }
+    __syncthreads();
     // Early-termination counts per context of the current plane (d = 0 low half, d = 1 high
     // half) and the contexts' entropy terms.
     __shared__ uint32_t s_hist[WAVES][2][32];
@@ -175,28 +214,29 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
         uint32_t sgn = 0, colmax = 0;
         {
             // all 32 loads in flight at once: rows and columns outside the block read the
-            // block's first sample (a valid address) and are discarded
+            // block's first sample (a valid address). What they quantise to is a value of the
+            // block, so it changes no maximum, and the passes mask it out; so do they the signs
+            // of samples that quantise to 0.
             const float* src = fr.coef + blk.coef_off + (x < w ? x : 0);
+            const float scale = band.inv_delta * 64.0f;  // a power of two apart: the same rounding
             float v[32];
 #pragma unroll
             for (int r = 0; r < 32; ++r) v[r] = src[(size_t)(r < h ? r : 0) * fr.stride];
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
-                const float a = (v[r] < 0.f ? -v[r] : v[r]) * band.inv_delta * 64.0f;
-                uint32_t q = a >= (float)band.max_mag ? band.max_mag : (uint32_t)a;
-                q = x < w && r < h ? q : 0u;
-                sgn |= (v[r] < 0.f && q >= 64u ? 1u : 0u) << r;
+            for (int r = 31; r >= 0; --r) {
+                uint32_t q;  // saturating, unlike the language's conversion
+                asm("v_cvt_u32_f32 %0, %1" : "=v"(q) : "v"(__builtin_fabsf(v[r]) * scale));
+                q = q < band.max_mag ? q : band.max_mag;
+                sgn = __builtin_amdgcn_alignbit(sgn, __float_as_uint(v[r]), 31);
                 m[r] = q;
                 colmax = q > colmax ? q : colmax;
             }
         }
         const uint32_t bmax = half_max_u(colmax) >> 6;
-        const int nbps = bmax ? 32 - __clz((int)bmax) : 0;
-        // the pair's plane and stripe counts, in scalar registers (wave-uniform loop bounds)
+        const int nbps = has && bmax ? 32 - __clz((int)bmax) : 0;
+        // the pair's plane count, in a scalar register (a wave-uniform loop bound)
         const int nbps_lo = __builtin_amdgcn_readlane(nbps, 0), nbps_hi = __builtin_amdgcn_readlane(nbps, 32);
         const int jmax = nbps_lo > nbps_hi ? nbps_lo : nbps_hi;
-        const int h_lo = __builtin_amdgcn_readlane(h, 0), h_hi = __builtin_amdgcn_readlane(h, 32);
-        const int nstripes = ((h_lo > h_hi ? h_lo : h_hi) + 3) >> 2;
         const uint32_t sgnL = from_left(sgn, x), sgnR = from_right(sgn, x);
         const uint32_t sgnU = sgn << 1, sgnD = sgn >> 1;
         const uint32_t rowsValid = h >= 32 ? 0xFFFFFFFFu : ((1u << h) - 1u);
@@ -223,7 +263,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
         auto window_sum = [&](uint32_t s) {
             int t = 0;
 #pragma unroll
-            for (int k = 0; k < 7; ++k) t += __popc(pl[k] & s) << k;
+            for (int k = 6; k >= 0; --k) t = 2 * t + __popc(pl[k] & s);
             return t;
         };
 
@@ -255,7 +295,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                 // refinement) symbol is written, keep1 those whose sign symbol is written,
                 // rl the run-length symbols of each stripe (a nibble per stripe); m0 / m1 the
                 // bits of those symbol bytes, one mask per bit.
-                uint32_t keep0 = 0, keep1 = 0, runs = 0, rl = 0, add0 = 0;
+                uint32_t keep0 = 0, keep1 = 0, runs = 0, rl = 0;
                 uint32_t m0[5] = {Bp, 0, 0, 0, 0}, m1[4] = {0, 0, 0, 0};
                 int dist = 0;
                 if (type == 1) {
@@ -265,10 +305,14 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                     keep0 = sig0 & colMask;
                     m0[1] = neighbour_any(S, SL, SR) & ~R;
                     m0[2] = R;
-                    add0 = 0x1C1C1C1Cu;
-                    // t1_dist_ref summed: 64 w - 5120 where bit p+6 is set, 3072 - 64 w elsewhere
-                    const uint32_t s1 = keep0 & Bp, s0 = keep0 & ~Bp;
-                    dist = 64 * window_sum(s1) - 5120 * __popc(s1) + 3072 * __popc(s0) - 64 * window_sum(s0);
+                    // t1_dist_ref summed: 64 w - 5120 where bit p+6 is set, 3072 - 64 w elsewhere.
+                    // A window bit counts for the first rows and against the others: the rows
+                    // where it equals bit p+6, less the others' number.
+                    const int ones = __popc(keep0 & Bp), zeros = __popc(keep0) - ones;
+                    int t = 0;
+#pragma unroll
+                    for (int k = 6; k >= 0; --k) t = 2 * t + __popc(keep0 & ~(pl[k] ^ Bp));
+                    dist = 64 * (t - 127 * zeros) - 5120 * ones + 3072 * zeros;
                     R |= keep0;
                 } else {
                     uint32_t N = 0;  // samples the pass turns significant
@@ -344,51 +388,45 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                         u3 = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
                     }
                     uint32_t base = plane_count;
-                    for (int s = 0; s < nstripes; ++s) {
-                        // this stripe's prefix and half-wave totals, then move the next ones up
-                        const uint32_t ex = e0 & 0xFFFFu, tlo = t0 & 0xFFFFu, thi = u0 & 0xFFFFu;
-                        {
-                            const uint32_t a = e0 >> 16, b = t0 >> 16, c = u0 >> 16;
-                            e0 = e1; e1 = e2; e2 = e3; e3 = a;
-                            t0 = t1; t1 = t2; t2 = t3; t3 = b;
-                            u0 = u1; u1 = u2; u2 = u3; u3 = c;
-                        }
+                    const uint32_t pre[4] = {e0, e1, e2, e3}, lo[4] = {t0, t1, t2, t3}, hi[4] = {u0, u1, u2, u3};
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) {
+                        // this stripe's prefix and half-wave totals
+                        const uint32_t ex = s < 4 ? pre[s & 3] & 0xFFFFu : pre[s & 3] >> 16;
+                        const uint32_t tlo = s < 4 ? lo[s & 3] & 0xFFFFu : lo[s & 3] >> 16;
+                        const uint32_t thi = s < 4 ? hi[s & 3] & 0xFFFFu : hi[s & 3] >> 16;
                         if (tlo + thi == 0) continue;
-                        uint32_t pos = base + ex;
+                        uint8_t* out = sym + base + ex;
                         base += half ? thi : tlo;
                         const int r0 = 4 * s;
-                        const uint32_t z = (keep0 >> r0) & 0xFu, gn = (keep1 >> r0) & 0xFu;
-                        const uint32_t w0 = add0 + (stripe_bytes(m0[0], r0) | stripe_bytes(m0[1], r0) << 1 |
-                                                    stripe_bytes(m0[2], r0) << 2 | stripe_bytes(m0[3], r0) << 3 |
-                                                    stripe_bytes(m0[4], r0) << 4);
-                        if (type == 2 && __any(((runs >> r0) & 1u) != 0)) {
-                            // run-length symbols: context 17 with whether a row turns
-                            // significant, then that row's position in two context-18 bits
-                            const bool run = (runs >> r0) & 1u, hit = run && gn != 0;
-                            const uint32_t first = gn ? (uint32_t)__builtin_ctz(gn) : 0u;
-                            *(run ? sym + pos : junk) = (uint8_t)(34u | (gn != 0));
-                            *(hit ? sym + pos + 1 : junk) = (uint8_t)(36u | (first >> 1));
-                            *(hit ? sym + pos + 2 : junk) = (uint8_t)(36u | (first & 1u));
-                            pos += run ? (hit ? 3u : 1u) : 0u;
-                        }
+                        const uint32_t z = (keep0 >> r0) & 0xFu;
                         if (type == 1) {
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const uint32_t zk = (z >> k) & 1u;
-                                *(zk ? sym + pos : junk) = (uint8_t)(w0 >> (8 * k));
-                                pos += zk;
-                            }
+                            const uint32_t w0 = 0x1C1C1C1Cu + stripe_bits(stripe_bits(stripe_bytes(m0[0], r0), m0[1], r0, 1),
+                                                                          m0[2], r0, 2);
+                            put_bytes(__builtin_amdgcn_perm(0u, w0, s_order[z].x), (uint32_t)__popc(z), out, junk);
                         } else {
-                            const uint32_t w1 = 0x12121212u + (stripe_bytes(m1[0], r0) | stripe_bytes(m1[1], r0) << 1 |
-                                                               stripe_bytes(m1[2], r0) << 2 | stripe_bytes(m1[3], r0) << 3);
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const uint32_t zk = (z >> k) & 1u, gk = (gn >> k) & 1u;
-                                *(zk ? sym + pos : junk) = (uint8_t)(w0 >> (8 * k));
-                                pos += zk;
-                                *(gk ? sym + pos : junk) = (uint8_t)(w1 >> (8 * k));
-                                pos += gk;
+                            const uint32_t gn = (keep1 >> r0) & 0xFu;
+                            if (type == 2 && __any(((runs >> r0) & 1u) != 0)) {
+                                // run-length symbols: context 17 with whether a row turns
+                                // significant, then that row's position in two context-18 bits
+                                const bool run = (runs >> r0) & 1u, hit = run && gn != 0;
+                                const uint32_t first = gn ? (uint32_t)__builtin_ctz(gn) : 0u;
+                                *(run ? out : junk) = (uint8_t)(34u | (gn != 0));
+                                uint8_t* const more = hit ? out : junk;
+                                more[1] = (uint8_t)(36u | (first >> 1));
+                                more[2] = (uint8_t)(36u | (first & 1u));
+                                out += run ? (hit ? 3u : 1u) : 0u;
                             }
+                            uint32_t w0 = stripe_bits(stripe_bytes(m0[3], r0), m0[4], r0, 1) << 3;
+                            w0 |= stripe_bits(stripe_bits(stripe_bytes(m0[0], r0), m0[1], r0, 1), m0[2], r0, 2);
+                            const uint32_t w1 =
+                                0x12121212u + (stripe_bits(stripe_bits(stripe_bytes(m1[0], r0), m1[1], r0, 1), m1[2], r0, 2) |
+                                               stripe_bytes(m1[3], r0) << 3);
+                            // the stripe's symbols in order, without gaps
+                            const uint2 order = s_order[z | gn << 4];
+                            const uint32_t n = (uint32_t)(__popc(z) + __popc(gn));
+                            put_bytes(__builtin_amdgcn_perm(w1, w0, order.x), n, out, junk);
+                            if (__any(n > 4u)) put_bytes(__builtin_amdgcn_perm(w1, w0, order.y), n > 4u ? n - 4u : 0u, out + 4, junk);
                         }
                     }
                     sym_total += base - plane_count;
@@ -416,17 +454,17 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                 plane_count += fill;
             }
             wave_sync();
-            // early-termination counts of the plane's symbols, 32 lanes per block at a time
-            // (not one lane per column inside the divergent emission loops)
+            // early-termination counts of the plane's symbols, 32 lanes per block at a time (not
+            // one lane per column inside the emission loops): per context the symbols, and the
+            // ones among them << 16. The plane is a multiple of 16 symbols long.
             if (track && act)
                 for (uint32_t i = 4u * (uint32_t)x; i < plane_count; i += 128u) {
                     const uint32_t w4 = *(const uint32_t*)(sym + i);  // within the staging area
 #pragma unroll
-                    for (uint32_t j = 0; j < 4; ++j)
-                        if (i + j < plane_count) {
-                            const uint32_t sv = w4 >> (8 * j);
-                            atomicAdd(&hist[(sv >> 1) & 31u], (sv & 1u) ? 0x10000u : 1u);
-                        }
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t at = (j ? w4 >> (8 * j - 1) : w4 << 1) & 0x7Cu;
+                        atomicAdd((uint32_t*)((char*)hist + at), ((w4 >> (8 * j)) & 1u) << 16 | 1u);
+                    }
                 }
             const uint32_t cnt_lo = __shfl((int)plane_count, 0), cnt_hi = __shfl((int)plane_count, 32);
             // 64-byte aligned: the MQ coder reads a plane in 64-byte groups
@@ -456,7 +494,7 @@ __global__ void __launch_bounds__(WAVES * 64, 3) t1_cm_kernel(CmParams P) {
                 float term = 0.f;
                 if (track && x < 19) {
                     const uint32_t hv = hist[x];
-                    const uint32_t n0 = hv & 0xFFFFu, n1 = hv >> 16, n = n0 + n1;
+                    const uint32_t n = hv & 0xFFFFu, n1 = hv >> 16, n0 = n - n1;
                     if (n > 0 && n <= kLog2Max) {
                         const float* row = P.log2tab + (size_t)n * (n + 1) / 2;
                         const float a = (float)n0 * row[n0];
