@@ -525,6 +525,14 @@ public:
     }
     double data(int c, int b) const { return (double)rate_[(size_t)c * (nb_ + 1) + b]; }
     double incl(int c, int b) const { return (double)incl_[(size_t)c * (nb_ + 1) + b]; }
+    template <class Ok> int first(int lo, int hi, const Ok& ok) const {
+        while (lo < hi) {
+            const int mid = lo + (hi - lo) / 2;
+            if (ok(mid)) hi = mid;
+            else lo = mid + 1;
+        }
+        return lo;
+    }
 
 private:
     struct Part {

@@ -169,7 +169,8 @@ size_t Job::estimateBytes(const std::vector<SlotCapacity>& slots, const JobOptio
     // one histogram per slot
     total += (size_t)n * (kMaxPasses * (8 + 8 + 4 + 4) + 4 + 4) + (size_t)nb * 8;
     total += 16 * rcPartEntries(n, slots.size()) + 4 * rc_segsum_entries(slots.size());
-    total += slots.size() * (6 * (size_t)(kRcMaxBins + 1) * 4 + sizeof(RcFrame));
+    total += slots.size() * (6 * (size_t)(kRcMaxBins + 1) * 4 + sizeof(RcFrame) + 8 * kRcDistSums) +
+             rc_run_bytes(slots.size());
     total += z.pool + z.out;
     return total;
 }
@@ -309,6 +310,8 @@ void Job::allocate() {
     dHullKbin_ = devAlloc<int32_t>((size_t)blockCap_ * kMaxPasses);
     dHullN_ = devAlloc<uint32_t>(blockCap_);
     dRcSel_ = devAlloc<uint32_t>(blockCap_);
+    dRcRuns_ = (RcRun*)devAlloc<uint8_t>(rc_run_bytes(ns));
+    dRcDist_ = devAlloc<unsigned long long>((size_t)ns * kRcDistSums);
     dRcPart_ = devAlloc<unsigned long long>(2 * rcPartEntries(blockCap_, ns));
     dRcSegsum_ = devAlloc<uint32_t>(rc_segsum_entries(ns));
     // the rate control leaves its histogram zero after every run; it starts zero
@@ -362,7 +365,7 @@ void Job::bind(std::vector<FrameConfig> frames) {
     uint32_t nblocks = 0, nbands = 0;
     int maxLevels = 0;
     bool anyRc = false;
-    uint32_t rcMaxBlocks = 0;
+    uint32_t rcMaxBlocks = 0, rcMaxPackets = 0;
     for (int f = 0; f < nf; ++f) {
         const FrameConfig& fc = frames[f];
         const Layout& L = fc.layout;
@@ -443,6 +446,7 @@ void Job::bind(std::vector<FrameConfig> frames) {
             for (int k = 0; k < 6; ++k) rc.tp_comp[k] = T.tpComp[k];
             anyRc = true;
             rcMaxBlocks = std::max(rcMaxBlocks, d.numBlocks);
+            rcMaxPackets = std::max(rcMaxPackets, rc.npackets);
         }
         nblocks += d.numBlocks;
         maxLevels = std::max(maxLevels, L.levels);
@@ -456,6 +460,7 @@ void Job::bind(std::vector<FrameConfig> frames) {
     hipCheck(hipMemcpyAsync(dRc_, hRc_, sizeof(RcFrame) * nf, hipMemcpyHostToDevice, s), "rate-control frames");
     anyRc_ = anyRc;
     rcMaxBlocks_ = rcMaxBlocks;
+    rcMaxPackets_ = rcMaxPackets;
     nblocks_ = nblocks;
     numLevels_ = maxLevels;
     frames_ = std::move(frames);
@@ -787,8 +792,10 @@ void Job::enqueueT1(hipStream_t s) {
         rp.mantissa = ctx_.octaveMantissa();
         rp.first = ctx_.octaveFirst();
         rp.sel = dRcSel_;
+        rp.runs = dRcRuns_;
+        rp.dist = dRcDist_;
         rp.counters = dCounters_;
-        hipCheck(launch_rc(rp, numFrames(), rcMaxBlocks_, s), "rate control");
+        hipCheck(launch_rc(rp, numFrames(), rcMaxBlocks_, rcMaxPackets_, s), "rate control");
     }
     hipCheck(launch_compact_offsets(dInfo_, dCodeLen_, n, dDataOff_, nullptr, dPartial_, s), "compaction offsets");
     // dense results live in the (now consumed) symbol pool

@@ -295,9 +295,12 @@ private:
     int32_t* dHullKbin_ = nullptr;
     uint32_t* dHullN_ = nullptr;
     uint32_t* dRcSel_ = nullptr;
+    RcRun* dRcRuns_ = nullptr;
+    unsigned long long* dRcDist_ = nullptr;
     unsigned long long* dRcPart_ = nullptr;
     uint32_t* dRcSegsum_ = nullptr;
     uint32_t rcMaxBlocks_ = 0;       // most blocks of a rate-controlled frame
+    uint32_t rcMaxPackets_ = 0;      // most packets of one
     uint32_t* dRcHist_ = nullptr;
     // Tier-1 arrays
     T1Info* dInfo_ = nullptr;

@@ -90,7 +90,7 @@ struct CompactParams {
 };
 
 // Device rate control (kernels_rc.hip), after MQ, before compaction: a hull launch over
-// every block, then one workgroup per frame.
+// every block and every packet, the search step by step in between.
 struct RcParams {
     RcFrame* frames;
     const T1Block* blocks;
@@ -112,13 +112,18 @@ struct RcParams {
     uint32_t* segsum;           // [rc_segsum_entries] scan segment totals
     const unsigned long long* mantissa;  // [1025] the octave's steps
     const uint16_t* first;               // [1024]
-    uint32_t* sel;              // [block] chosen passes << 24 | their length
+    uint32_t* sel;              // [block] hull points kept
+    struct RcRun* runs;         // [frame] the search between its launches
+    unsigned long long* dist;   // [frame][kRcDistSums] partial sums (doubles) of the distortion left
     const JobCounters* counters;
 };
+constexpr int kRcDistSums = 1024;
+size_t rc_run_bytes(size_t frames);
 // Entries of RcParams::part for a job of `blocks` code-blocks in `frames` frames.
 inline size_t rcPartEntries(size_t blocks, size_t frames) { return blocks / 256 + frames + 2; }
 size_t rc_segsum_entries(size_t frames);
-hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, hipStream_t s);
+hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, uint32_t max_frame_packets,
+                     hipStream_t s);
 
 hipError_t launch_dwt_level(bool level0, int tile_shape, const DwtLevelDesc* descs, int ndesc, int tiles,
                             hipStream_t s);

@@ -11,12 +11,13 @@
 //   rc_fill_kernel   one thread per code-block: the slope histogram (bytes and included
 //                    blocks per component, 32-bit integer atomics);
 //   rc_scan_kernel   two passes over 1,024-bin segments: suffix sums of the histogram;
-//   rc_kernel        one 1024-thread workgroup per frame: the lambda search of rc_shared.h
-//                    in thread 0; each size measurement selects every block's passes (and
-//                    writes them, with their length, over the block's pass count and
-//                    codeword length, which compaction uses) and sizes every packet
-//                    (rc_packet_bytes, in registers), the tile-part sums in LDS. At the end
-//                    it clears the histogram bins it used, so every run finds them zero.
+//   rc_measure_kernel  a few times: a size measurement of every frame, one wave per packet
+//                    (its blocks' choices, then its exact size), the tile-part sums in global
+//                    memory; the workgroup that is last to finish a frame runs one step of the
+//                    search of rc_shared.h. A frame whose search is over does nothing.
+//   rc_finish_kernel one workgroup per frame: any further steps of the search, and the result;
+//   rc_dist_kernel   the distortion left, and the histogram bins the run used cleared, so that
+//                    every run finds them zero.
 //
 // The host library runs the same shared code, so both choose the same passes.
 #include <hip/hip_runtime.h>
@@ -27,13 +28,31 @@
 
 namespace gail_amd {
 
+// A frame's search between the launches of a run.
+struct RcRun {
+    RcSearch search;
+    unsigned long long tp[6];  // tile-part bytes of the measurement under way
+    uint32_t arrived;          // its workgroups that are through
+    uint32_t done;
+    uint32_t summed;           // workgroups of rc_dist_kernel that are through
+};
+
 namespace {
+
+// LDS written by other lanes of the wave is read after this.
+__device__ __forceinline__ void lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 constexpr int kHullThreads = 256;  // blocks per hull / fill workgroup (one partial slope range each)
 constexpr int kScanThreads = 256;
 constexpr int kScanBins = 4 * kScanThreads;  // bins per scan workgroup
 constexpr int kScanSegs = (kRcMaxBins + 1 + kScanBins - 1) / kScanBins;
-constexpr int kRcThreads = 1024;
+constexpr int kMeasureWaves = 4;   // packets per workgroup of a measurement
+constexpr int kFinishWaves = 16;
+constexpr int kMeasureLaunches = 6;
 constexpr int32_t kBinAbove = 0x7FFFFFFF;      // slope bin of an infinite slope
 constexpr int32_t kBinBelow = -0x7FFFFFFF - 1;  // of a slope <= 0
 
@@ -46,26 +65,27 @@ __device__ __forceinline__ uint32_t part_index(const RcFrame& F, uint32_t f, uin
     return F.first_block / kHullThreads + f + x;
 }
 
-// RcSearch reads the histogram sums through data(c, b) and incl(c, b).
+// RcSearch's view of the histogram sums, for a whole wave that runs the search with the same
+// values in every lane.
 struct DevHistView {
     const uint32_t* rate[3];
-    const uint32_t* incl[3];
+    const uint32_t* incl_[3];
     __device__ double data(int c, int b) const { return (double)rate[c][b]; }
-    __device__ double incl_(int c, int b) const { return (double)incl[c][b]; }
-};
-struct DevHistRef {
-    const DevHistView* h;
-    __device__ double data(int c, int b) const { return h->data(c, b); }
-    __device__ double incl(int c, int b) const { return h->incl_(c, b); }
-};
-
-// Frame-local view of the blocks for rc_packet_bytes: sel = passes << 24 | length.
-struct DevBlocks {
-    const uint32_t* sel;   // + first block
-    const T1Info* info;    // + first block
-    __device__ uint32_t passes(uint32_t i) const { return sel[i] >> 24; }
-    __device__ uint32_t len(uint32_t i) const { return sel[i] & 0xFFFFFFu; }
-    __device__ uint32_t nbps(uint32_t i) const { return info[i].nbps; }
+    __device__ double incl(int c, int b) const { return (double)incl_[c][b]; }
+    // 64 probes at once: 3 rounds of loads for 65,536 bins instead of a chain of 16
+    template <class Ok> __device__ int first(int lo, int hi, const Ok& ok) const {
+        const int lane = threadIdx.x & 63;
+        while (lo < hi) {
+            const int step = (hi - lo + 63) / 64;
+            const int at = lo + (lane + 1) * step - 1;
+            const unsigned long long m = __ballot(at >= hi || ok(at));
+            if (!m) return hi;
+            const int l = __ffsll(m) - 1;
+            hi = min(hi, lo + (l + 1) * step - 1);
+            lo += l * step;
+        }
+        return lo;
+    }
 };
 
 // Point-major hull store of one block.
@@ -167,6 +187,22 @@ __global__ void __launch_bounds__(kHullThreads) rc_range_kernel(RcParams P) {
         F.nb = nb;
         F.min_slope = mn;
         F.max_slope = mx;
+        RcRun& R = P.runs[f];
+        RcSearch S{};
+        S.init();
+        S.kLo = kLo;
+        S.nb = nb;
+        S.minSlope = mn;
+        S.maxSlope = mx;
+        S.maxTotal = F.max_total;
+        S.maxComp = F.max_comp;
+        S.mantissa = P.mantissa;
+        S.first = P.first;
+        R.search = S;
+        for (int k = 0; k < 6; ++k) R.tp[k] = 0;
+        R.arrived = 0;
+        R.done = 0;
+        R.summed = 0;
     }
 }
 
@@ -258,124 +294,353 @@ __global__ void __launch_bounds__(kScanThreads) rc_scan_kernel(RcParams P) {
         if (b0 + j < n1) v[b0 + j] = x[j] + carry;
 }
 
-__global__ void __launch_bounds__(kRcThreads) rc_kernel(RcParams P) {
+namespace {
+
+// Waits for an atomic that returned v: what the device-scope atomics of a workgroup's other waves
+// and of later ones read is then in place, without the write-back of the whole L2 that a
+// device-scope fence costs (a measurement of 16 4K frames 285 us with fences, 50 without).
+__device__ __forceinline__ void atomic_done(unsigned long long v) {
+    asm volatile("" ::"v"((uint32_t)v), "v"((uint32_t)(v >> 32)) : "memory");
+}
+
+// Bits of the longest packet header: 48 blocks of at most 3 inclusion bits, 258 for the zero
+// bit-planes (Mb fits in 8 bits), 16 for the passes, 22 for Lblock and 29 for the length.
+constexpr int kHeaderWords = 512;
+
+// The bits v (below 1 << n, n <= 32) at bit `at` of a string whose bit 0 is word 0's highest.
+__device__ __forceinline__ void put_bits(uint32_t* words, uint32_t at, uint32_t v, uint32_t n) {
+    if (!v) return;  // the string is zero before
+    const unsigned long long w = (unsigned long long)v << (64u - n - (at & 31u));
+    const uint32_t hi = (uint32_t)(w >> 32), lo = (uint32_t)w;
+    if (hi) atomicOr(words + (at >> 5), hi);
+    if (lo) atomicOr(words + (at >> 5) + 1, lo);
+}
+
+// One packet at thresholds lambda, by a whole wave: lane q of each group of 16 chooses the
+// passes of leaf q of one precinct-band and writes its part of the header; returns the
+// packet's bytes (rc_packet_bytes of the same choices) in every lane.
+//
+// A hull's slopes fall strictly, so its points of slope >= lambda are a prefix: their number
+// is counted, eight at a time. The choice and its length replace the block's pass
+// count and codeword length at once (the last measurement's stay).
+__device__ unsigned long long measure_packet(const RcParams& P, const RcFrame& F, uint32_t k, const double lambda[3],
+                                             uint32_t* words) {
+    const int lane = threadIdx.x & 63, q = lane & 15, group = lane >> 4;
+    const RcPacket pk = F.packets[k];
+    const bool band = group < pk.nband;
+    const RcPBand pb = F.pbands[pk.first + (band ? group : 0)];
+    const int w = band ? pb.ncbx : 0, h = band ? pb.ncby : 0;
+    const bool leaf = (q & 3) < w && (q >> 2) < h;
+    uint32_t np = 0, len = 0;
+    int zv = 255;
+    if (leaf) {
+        const uint32_t cb = F.first_block + pb.block0 + (uint32_t)(q >> 2) * pb.stride + (uint32_t)(q & 3);
+        const uint32_t hn = P.hull_n[cb], nbps = P.info[cb].nbps;
+        const uint32_t cnt = hn & 0xFFu, c = hn >> 8;
+        const double lam = c == 0 ? lambda[0] : c == 1 ? lambda[1] : lambda[2];
+        uint32_t kept = 0;
+        for (uint32_t i = 0; i < cnt; i += 8) {  // eight points' loads in flight at once
+            double s[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) s[j] = P.h_slope[(size_t)(i + j < cnt ? i + j : i) * P.stride + cb];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) kept += i + j < cnt && s[j] >= lam;
+            if (kept < i + 8) break;
+        }
+        const uint32_t sel = kept ? P.h_sel[(size_t)(kept - 1) * P.stride + cb] : 0u;
+        np = sel >> 24;
+        len = sel & 0xFFFFFFu;
+        zv = (int)pb.mb - (int)nbps;
+        P.sel[cb] = kept;
+        P.info[cb].passes = np;
+        P.code_len[cb] = len;
+    }
+    const unsigned long long included = __ballot(np != 0);
+    if (!included) return 1;  // an empty packet is one zero byte
+
+    // The band's tag trees (rc_packet_code): which lane meets each node first, in leaf order.
+    const uint32_t incl = (uint32_t)(included >> (lane & 48)) & 0xFFFFu;
+    const int levels = (w == 1 && h == 1) ? 1 : ((w <= 2 && h <= 2) ? 2 : 3);
+    const int qm = (q >> 3) * 8 + ((q >> 1) & 1) * 2;  // the quad's first leaf
+    const uint32_t quad = incl & (0x33u << qm);
+    int zq = min(zv, __shfl_xor(zv, 1));
+    zq = min(zq, __shfl_xor(zq, 4));
+    int zroot = min(zq, __shfl_xor(zq, 2));
+    zroot = min(zroot, __shfl_xor(zroot, 8));
+    uint32_t ibits = 0, icount = 0;  // inclusion
+    if (leaf) {
+        bool go = true;
+        if (levels >= 2) {
+            go = incl != 0;
+            if (q == 0) {
+                ibits = go;
+                icount = 1;
+            }
+        }
+        if (go && levels == 3) {
+            go = quad != 0;
+            if (q == qm) {
+                ibits = ibits << 1 | (go ? 1u : 0u);
+                ++icount;
+            }
+        }
+        if (go) {
+            ibits = ibits << 1 | (np ? 1u : 0u);
+            ++icount;
+        }
+    }
+    // zero bit-planes: at each node met first, (value - parent's value) zeros and a one
+    uint32_t zr = 0, zn = 0, zl = 0, pbits = 0, pcount = 0, lcount = 0, incr = 0;
+    if (np) {
+        const uint32_t before = incl & ((1u << q) - 1u);
+        int prev = 0;
+        if (levels >= 2) {
+            if (!before) zr = (uint32_t)max(zroot - prev + 1, 0);
+            prev = zroot;
+        }
+        if (levels == 3) {
+            if (!(before & quad)) zn = (uint32_t)max(zq - prev + 1, 0);
+            prev = zq;
+        }
+        zl = (uint32_t)max(zv - prev + 1, 0);
+        // Table B.4: codewords for the number of coding passes
+        pbits = np == 1 ? 0u : np == 2 ? 2u : np <= 5 ? 0xCu | (np - 3) : np <= 36 ? 0x1E0u | (np - 6) : 0xFF80u | (np - 37);
+        pcount = np == 1 ? 1u : np == 2 ? 2u : np <= 5 ? 4u : np <= 36 ? 9u : 16u;
+        const uint32_t extra = (uint32_t)rc_floor_log2(np), need = len ? (uint32_t)rc_floor_log2(len) + 1 : 1u;
+        incr = need > 3 + extra ? need - (3 + extra) : 0u;
+        lcount = 3 + incr + extra;
+    }
+    const uint32_t bits = icount + zr + zn + zl + pcount + (np ? incr + 1 : 0u) + lcount;
+    uint32_t end = bits, body = len;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t e = (uint32_t)__shfl_up((int)end, o), b = (uint32_t)__shfl_up((int)body, o);
+        if (lane >= o) {
+            end += e;
+            body += b;
+        }
+    }
+    const uint32_t total = 1u + (uint32_t)__shfl((int)end, 63);  // the leading 1: not empty
+    const unsigned long long bytes = (uint32_t)__shfl((int)body, 63);
+
+    // the header as one bit string, without the bits that marker stuffing adds
+    for (uint32_t i = lane; i <= (total + 63) / 32; i += 64) words[i] = 0;
+    lds_sync();
+    uint32_t at = 1u + end - bits;
+    if (lane == 0) put_bits(words, 0, 1, 1);
+    put_bits(words, at, ibits, icount);
+    at += icount;
+    if (np) {
+        if (zr) put_bits(words, at += zr - 1, 1, 1), ++at;
+        if (zn) put_bits(words, at += zn - 1, 1, 1), ++at;
+        if (zl) put_bits(words, at += zl - 1, 1, 1), ++at;
+        put_bits(words, at, pbits, pcount);
+        at += pcount;
+        put_bits(words, at, ((1u << incr) - 1u) << 1, incr + 1);
+        at += incr + 1;
+        put_bits(words, at, len, lcount);
+    }
+    lds_sync();
+    // A byte after 0xFF holds 7 bits: from each start, 64 bytes at a time, to the next 0xFF.
+    uint32_t pos = 0, count = 0;
+    for (;;) {
+        const uint32_t p = pos + 8u * (uint32_t)lane;
+        uint32_t byte = 0;
+        if (p + 8 <= total) {
+            const unsigned long long v = (unsigned long long)words[p >> 5] << 32 | words[(p >> 5) + 1];
+            byte = (uint32_t)(v >> (56u - (p & 31u))) & 0xFFu;
+        }
+        const unsigned long long ff = __ballot(byte == 0xFFu);
+        if (ff) {
+            const uint32_t n = (uint32_t)__ffsll(ff);
+            pos += 8 * n + 7;
+            count += n + 1;  // with the 7-bit byte that follows, full or padded or empty
+        } else {
+            const uint32_t left = pos < total ? (total - pos + 7) / 8 : 0u;
+            const uint32_t n = left < 64 ? left : 64;
+            pos += 8 * n;
+            count += n;
+        }
+        if (pos >= total) break;
+    }
+    return bytes + count;
+}
+
+// One step of a frame's search by a whole wave, after a measurement whose tile-part sums are
+// tp; returns whether another is wanted and leaves the state for it.
+__device__ bool search_step(const RcParams& P, uint32_t f, RcFrame& F, const unsigned long long tp[6]) {
+    RcRun& R = P.runs[f];
+    RcSearch S = R.search;
+    DevHistView H;
+    for (int c = 0; c < 3; ++c) {
+        H.rate[c] = hist_of(P, f, c);
+        H.incl_[c] = hist_of(P, f, 3 + c);
+    }
+    RcSizes sz;
+    sz.total = F.fixed_bytes;
+    sz.comp[0] = sz.comp[1] = sz.comp[2] = 0;
+    for (uint32_t k = 0; k < F.ntp; ++k) {
+        const unsigned long long b = tp[k] + 14;  // SOT + SOD of each tile-part
+        const int c = F.tp_comp[k];
+        sz.comp[0] += c == 0 ? b : 0;
+        sz.comp[1] += c == 1 ? b : 0;
+        sz.comp[2] += c == 2 ? b : 0;
+        sz.total += b;
+    }
+    const bool more = S.next(H, sz);
+    if ((threadIdx.x & 63) == 0) {
+        R.search = S;
+        R.done = more ? 0u : 1u;
+        R.arrived = 0;
+        for (int k = 0; k < 6; ++k) R.tp[k] = 0;
+        if (!more) {
+            for (int c = 0; c < 3; ++c) F.lambda[c] = S.lambda[c];
+            F.total = sz.total;
+            for (int c = 0; c < 3; ++c) F.comp[c] = sz.comp[c];
+            for (uint32_t k = 0; k < 6; ++k) F.tile_part[k] = k < F.ntp ? tp[k] + 14 : 0ull;
+            F.iterations = S.iterations;
+            F.status = 0;
+        }
+    }
+    return more;
+}
+
+}  // namespace
+
+// Bound by latency: the loads of a block's hull, the scan of its packet's header bits and the
+// search's probes, one after the other. One 4K frame has some 600 packets, a wave each. With
+// one workgroup per frame for the whole search (a thread per packet's header, 26 blocks a
+// thread, a thread's chain of 16 probes) a search of three measurements took 615 us for one 4K
+// frame and 660 for 16; these launches with the finish and distortion kernels take 97 and 190.
+// Frames with one budget take 3 or 4 measurements, those held by a component's cap 5 and more:
+// six launches, each 4 us when there is nothing left to do (24 us otherwise); further steps run
+// in rc_finish_kernel at 180 us each.
+__global__ void __launch_bounds__(kMeasureWaves * 64) rc_measure_kernel(RcParams P) {
+    __shared__ uint32_t s_words[kMeasureWaves][kHeaderWords];
+    __shared__ uint32_t s_last;
+    const uint32_t f = blockIdx.y;
+    RcFrame& F = P.frames[f];
+    if (F.max_total == 0) return;
+    if (P.counters->flags & 3u) return;
+    RcRun& R = P.runs[f];
+    const uint32_t groups = (F.npackets + kMeasureWaves - 1) / kMeasureWaves;
+    if (R.done || blockIdx.x >= groups) return;
+    const uint32_t wv = threadIdx.x >> 6, k = blockIdx.x * kMeasureWaves + wv;
+    const double lambda[3] = {R.search.lambda[0], R.search.lambda[1], R.search.lambda[2]};
+    if (k < F.npackets) {
+        const unsigned long long b = measure_packet(P, F, k, lambda, s_words[wv]);
+        if ((threadIdx.x & 63) == 0) atomic_done(atomicAdd(&R.tp[F.packets[k].tp], b));
+    }
+    // the state is read above by every wave before the last workgroup to arrive replaces it
+    __syncthreads();
+    if (threadIdx.x == 0) s_last = atomicAdd(&R.arrived, 1u) == groups - 1;
+    __syncthreads();
+    if (!s_last || wv != 0) return;
+    unsigned long long tp[6];
+    for (int i = 0; i < 6; ++i) tp[i] = __hip_atomic_load(&R.tp[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    search_step(P, f, F, tp);
+}
+
+__global__ void __launch_bounds__(kFinishWaves * 64) rc_finish_kernel(RcParams P) {
+    __shared__ uint32_t s_words[kFinishWaves][kHeaderWords];
     __shared__ unsigned long long s_tp[6];
-    __shared__ double s_lambda[3];
-    __shared__ double s_dist[kRcThreads];
-    __shared__ int s_more;
+    __shared__ uint32_t s_more;
     const uint32_t f = blockIdx.x;
     RcFrame& F = P.frames[f];
     if (F.max_total == 0) return;
     if (P.counters->flags & 3u) return;
-    const int t = threadIdx.x;
-    const uint32_t n = F.nblocks, b0 = F.first_block;
-    const int nb = F.nb;
-
-    RcSearch S;  // thread 0's
-    if (t == 0) {
-        S.init();
-        S.kLo = F.k_lo;
-        S.nb = nb;
-        S.minSlope = F.min_slope;
-        S.maxSlope = F.max_slope;
-        S.maxTotal = F.max_total;
-        S.maxComp = F.max_comp;
-        S.mantissa = P.mantissa;
-        S.first = P.first;
-        for (int c = 0; c < 3; ++c) s_lambda[c] = 0.0;
-    }
-    __syncthreads();
-    DevHistView H;
-    for (int c = 0; c < 3; ++c) {
-        H.rate[c] = hist_of(P, f, c);
-        H.incl[c] = hist_of(P, f, 3 + c);
-    }
-    const DevHistRef HV{&H};
-    const DevBlocks blk{P.sel + b0, P.info + b0};
-
-    // ---- measure, search, measure ... (thread 0 decides, everyone measures)
-    double dist = 0;
+    RcRun& R = P.runs[f];
+    if (R.done) return;
+    const uint32_t wv = threadIdx.x >> 6;
     for (;;) {
-        // A hull's slopes fall strictly, so its points of slope >= lambda are a prefix and
-        // the last of them (rc_select) is found without a data-dependent exit. The choice
-        // and its length replace the block's pass count and codeword length at once (the
-        // last measurement's stay); dist sums the gains of the points left out.
-        dist = 0;
-        for (uint32_t i = t; i < n; i += kRcThreads) {
-            const uint32_t cb = b0 + i;
-            const uint32_t hn = P.hull_n[cb];
-            const uint32_t cnt = hn & 0xFFu;
-            const double lam = s_lambda[hn >> 8];
-            uint32_t sel = 0;
-            for (uint32_t h = 0; h < cnt; h += 4) {  // four points' loads in flight at once
-                double s[4], g[4];
-                uint32_t hs[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const size_t at = (size_t)(h + j) * P.stride + cb;
-                    const bool in = h + j < cnt;
-                    s[j] = in ? P.h_slope[at] : 0.0;
-                    g[j] = in ? P.h_gain[at] : 0.0;
-                    hs[j] = in ? P.h_sel[at] : 0u;
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (h + j < cnt) {
-                        if (s[j] >= lam) sel = hs[j];
-                        else dist += g[j];
-                    }
-            }
-            P.sel[cb] = sel;
-            P.info[cb].passes = sel >> 24;
-            P.code_len[cb] = sel & 0xFFFFFFu;
-        }
-        if (t < 6) s_tp[t] = t < (int)F.ntp ? 14ull : 0ull;  // SOT + SOD of each tile-part
+        const double lambda[3] = {R.search.lambda[0], R.search.lambda[1], R.search.lambda[2]};
+        if (threadIdx.x < 6) s_tp[threadIdx.x] = 0;
         __syncthreads();
-        for (uint32_t k = t; k < F.npackets; k += kRcThreads) {
-            const RcPacket pk = F.packets[k];
-            atomicAdd(&s_tp[pk.tp], rc_packet_bytes(pk, F.pbands, blk));
+        for (uint32_t k = wv; k < F.npackets; k += kFinishWaves) {
+            const unsigned long long b = measure_packet(P, F, k, lambda, s_words[wv]);
+            if ((threadIdx.x & 63) == 0) atomicAdd(&s_tp[F.packets[k].tp], b);
         }
         __syncthreads();
-        if (t == 0) {
-            RcSizes sz;
-            sz.total = F.fixed_bytes;
-            sz.comp[0] = sz.comp[1] = sz.comp[2] = 0;
-            for (uint32_t k = 0; k < F.ntp; ++k) {
-                sz.comp[F.tp_comp[k]] += s_tp[k];
-                sz.total += s_tp[k];
-            }
-            const bool more = S.next(HV, sz);
-            s_more = more ? 1 : 0;
-            if (more)
-                for (int c = 0; c < 3; ++c) s_lambda[c] = S.lambda[c];
-            else {
-                for (int c = 0; c < 3; ++c) F.lambda[c] = S.lambda[c];
-                F.total = sz.total;
-                for (int c = 0; c < 3; ++c) F.comp[c] = sz.comp[c];
-                for (uint32_t k = 0; k < 6; ++k) F.tile_part[k] = k < F.ntp ? s_tp[k] : 0ull;
-                F.iterations = S.iterations;
-                F.status = 0;
-            }
+        if (wv == 0) {
+            unsigned long long tp[6];
+            for (int i = 0; i < 6; ++i) tp[i] = s_tp[i];
+            const bool more = search_step(P, f, F, tp);
+            if (threadIdx.x == 0) s_more = more;
         }
+        __threadfence_block();
         __syncthreads();
         if (!s_more) break;
     }
-
-    // ---- distortion left (fixed-order tree sum), and a clean histogram for the next run
-    s_dist[t] = dist;
-    __syncthreads();
-    for (int w = kRcThreads / 2; w > 0; w >>= 1) {
-        if (t < w) s_dist[t] += s_dist[t + w];
-        __syncthreads();
-    }
-    if (t == 0) F.distortion = s_dist[0];
-    for (int a = 0; a < 6; ++a) {
-        uint32_t* v = hist_of(P, f, a);
-        for (int b = t; b <= nb; b += kRcThreads) v[b] = 0u;
-    }
 }
 
-hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, hipStream_t s) {
+// The distortion left: the gains of the points left out, summed by 1,024 threads over blocks
+// t, t + 1024, ... in turn and then as a tree, an order that does not depend on the launch.
+__global__ void __launch_bounds__(kHullThreads) rc_dist_kernel(RcParams P) {
+    const uint32_t f = blockIdx.y;
+    RcFrame& F = P.frames[f];
+    if (F.max_total == 0) return;
+    if (P.counters->flags & 3u) return;
+    constexpr uint32_t groups = kRcDistSums / 64;
+    if (threadIdx.x >= 64) {  // the other waves clear the histogram
+        const uint32_t i0 = blockIdx.x * (kHullThreads - 64) + threadIdx.x - 64, step = groups * (kHullThreads - 64);
+        for (int a = 0; a < 6; ++a) {
+            uint32_t* v = hist_of(P, f, a);
+            for (uint32_t b = i0; b <= (uint32_t)F.nb; b += step) v[b] = 0u;
+        }
+        return;
+    }
+    const uint32_t t = blockIdx.x * 64 + threadIdx.x, n = F.nblocks;
+    double dist = 0;
+    for (uint32_t i = t; i < n; i += 4 * kRcDistSums) {
+        uint32_t from[4], to[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t at = i + j * kRcDistSums, cb = F.first_block + (at < n ? at : i);
+            from[j] = P.sel[cb];
+            to[j] = at < n ? P.hull_n[cb] & 0xFFu : 0u;
+        }
+        double g[4][4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                g[j][k] = from[j] + k < to[j]
+                              ? P.h_gain[(size_t)(from[j] + k) * P.stride + F.first_block + i + j * kRcDistSums]
+                              : 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) dist += g[j][k];
+            const size_t cb = (size_t)F.first_block + i + j * kRcDistSums;
+            for (uint32_t h = from[j] + 4; h < to[j]; h += 4) {
+                double r[4];
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) r[k] = h + k < to[j] ? P.h_gain[(size_t)(h + k) * P.stride + cb] : 0.0;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) dist += r[k];
+            }
+        }
+    }
+    unsigned long long* sums = P.dist + (size_t)f * kRcDistSums;
+    atomic_done(atomicExch(&sums[t], __builtin_bit_cast(unsigned long long, dist)));
+    uint32_t last = 0;
+    if (threadIdx.x == 0) last = atomicAdd(&P.runs[f].summed, 1u) == groups - 1;
+    if (!__shfl((int)last, 0)) return;
+    double s[groups];
+#pragma unroll
+    for (uint32_t k = 0; k < groups; ++k)
+        s[k] = __builtin_bit_cast(double, __hip_atomic_load(&sums[64 * k + threadIdx.x], __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+    for (uint32_t w = groups / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (uint32_t k = 0; k < w; ++k) s[k] += s[k + w];
+    for (int w = 32; w > 0; w >>= 1) s[0] += __shfl_down(s[0], w);
+    if (threadIdx.x == 0) F.distortion = s[0];
+}
+
+hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, uint32_t max_frame_packets,
+                     hipStream_t s) {
     const uint32_t gx = (max_frame_blocks + kHullThreads - 1) / kHullThreads;
     if (!gx || !frames) return hipSuccess;
     hipLaunchKernelGGL(rc_hull_kernel, dim3(gx, frames), dim3(kHullThreads), 0, s, p);
@@ -383,9 +648,15 @@ hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, h
     hipLaunchKernelGGL(rc_fill_kernel, dim3(gx, frames), dim3(kHullThreads), 0, s, p);
     hipLaunchKernelGGL(rc_scan_kernel<0>, dim3(kScanSegs, 6, frames), dim3(kScanThreads), 0, s, p);
     hipLaunchKernelGGL(rc_scan_kernel<1>, dim3(kScanSegs, 6, frames), dim3(kScanThreads), 0, s, p);
-    hipLaunchKernelGGL(rc_kernel, dim3(frames), dim3(kRcThreads), 0, s, p);
+    const uint32_t px = (max_frame_packets + kMeasureWaves - 1) / kMeasureWaves;
+    for (int i = 0; px && i < kMeasureLaunches; ++i)
+        hipLaunchKernelGGL(rc_measure_kernel, dim3(px, frames), dim3(kMeasureWaves * 64), 0, s, p);
+    hipLaunchKernelGGL(rc_finish_kernel, dim3(frames), dim3(kFinishWaves * 64), 0, s, p);
+    hipLaunchKernelGGL(rc_dist_kernel, dim3(kRcDistSums / 64, frames), dim3(kHullThreads), 0, s, p);
     return hipGetLastError();
 }
+
+size_t rc_run_bytes(size_t frames) { return frames * sizeof(RcRun); }
 
 size_t rc_segsum_entries(size_t frames) { return frames * 6 * kScanSegs; }
 

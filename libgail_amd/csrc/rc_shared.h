@@ -1,9 +1,9 @@
 // PCRD-opt rate control written once for the host and the GPU (rate_control.cpp:11-279,
 // t2.cpp:31-115): the rate-distortion hull of a code-block, the exact Tier-2 size of one
 // packet, and the lambda search as a state machine that asks for size measurements. The
-// host library runs it sequentially; the device runs it with one workgroup per frame, the
-// measurements spread over the workgroup. Both do every floating-point step in the same
-// order (no contraction), so they make the same choices.
+// host library runs it sequentially; the device spreads each measurement over the chip, a
+// wave per packet, and runs the search in one wave. Both do every floating-point step in the
+// same order (no contraction), so they make the same choices.
 #pragma once
 #include <cstdint>
 
@@ -326,7 +326,10 @@ GAIL_HD unsigned long long rc_packet_bytes(const RcPacket& P, const RcPBand* pba
 // last measurement gave (the first call: with every pass included) and returns true with
 // lambda[] set when it wants another measurement, false when it is done. Histogram sums
 // (bytes and included blocks per component, suffix sums over bins 0..nb) are read
-// through data(c, b) / incl(c, b) of H.
+// through data(c, b) / incl(c, b) of H, and H's first(lo, hi, ok) finds the smallest i in
+// [lo, hi] with ok(i), given that ok never turns false again as i grows and that hi counts
+// as ok: the sums fall with the bin and rounding keeps their order, so the way there (halving on the host, 64
+// probes at once on the device) does not matter.
 struct RcSizes {
     unsigned long long total, comp[3];
 };
@@ -379,24 +382,16 @@ struct RcSearch {
     }
     // smallest bin in [lo, nb] whose model meets the budget (all components, or component cc)
     template <class H> GAIL_HD int search(const H& h, int cc, int lo) const {
-        int hi = nb;
-        while (lo < hi) {
-            const int mid = lo + (hi - lo) / 2;
-            int bb[3] = {bin[0], bin[1], bin[2]};
+        return h.first(lo, nb, [&](int b) {
             double comp[3];
-            bool ok;
             if (cc < 0) {
-                bb[0] = bb[1] = bb[2] = mid;
-                ok = model(h, bb, comp) <= (double)maxTotal;
-            } else {
-                bb[cc] = mid;
-                model(h, bb, comp);
-                ok = comp[cc] <= (double)maxComp;
+                const int bb[3] = {b, b, b};
+                return model(h, bb, comp) <= (double)maxTotal;
             }
-            if (ok) hi = mid;
-            else lo = mid + 1;
-        }
-        return lo;
+            const int bb[3] = {cc == 0 ? b : bin[0], cc == 1 ? b : bin[1], cc == 2 ? b : bin[2]};
+            model(h, bb, comp);
+            return (cc == 0 ? comp[0] : cc == 1 ? comp[1] : comp[2]) <= (double)maxComp;
+        });
     }
 
     // Stages: 0 after the first measurement; 1 after a measurement of the main rounds;
