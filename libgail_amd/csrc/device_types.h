@@ -63,7 +63,8 @@ struct JobCounters {
     uint32_t flags;               // 1: symbol pool full, 2: codeword buffer full
     uint32_t pad;
     unsigned long long symbols;   // Tier-1 symbols of the job
-    uint32_t pad2[10];
+    unsigned long long kept;      // bytes kept, and passes << 36
+    uint32_t pad2[8];
 };
 
 // ---------------------------------------------------------------- rate control on the device

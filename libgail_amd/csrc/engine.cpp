@@ -325,10 +325,10 @@ void Job::allocate() {
     dChunks_ = devAlloc<uint2>((size_t)n * kMaxPlanes);
     dSnaps_ = devAlloc<MqSnapshot>((size_t)n * kMaxPasses);
     dPerm_ = devAlloc<uint32_t>(n);
-    dHist_ = devAlloc<uint32_t>(128);
+    dOrder_ = devAlloc<uint32_t>(kOrderWords);
     dOutOff_ = devAlloc<unsigned long long>(n);
     dDataOff_ = devAlloc<unsigned long long>(n);
-    dPartial_ = devAlloc<unsigned long long>(n / 2048 + 4);
+    dPartial_ = devAlloc<unsigned long long>(n / kPlanGroupBlocks + 4);
     dCodeLen_ = devAlloc<uint32_t>(n);
     dCounters_ = devAlloc<JobCounters>(1);
     dWork_ = devAlloc<uint32_t>(4);
@@ -721,7 +721,7 @@ void Job::uploadAsync(int i) {
 
 void Job::enqueueT1(hipStream_t s) {
     const uint32_t n = nblocks_;
-    hipCheck(launch_clear_counters(dCounters_, dWork_, 4, s), "clear counters");
+    hipCheck(launch_clear_counters(dCounters_, dWork_, 4, dOrder_, s), "clear counters");
     CmParams cm{};
     cm.blocks = dBlocks_;
     cm.bands = dBands_;
@@ -742,8 +742,7 @@ void Job::enqueueT1(hipStream_t s) {
         1, std::min<uint32_t>((pairs + waves - 1) / waves, (uint32_t)(ctx_.computeUnits() * opt_.cmGroupsPerCU)));
     hipCheck(launch_t1_cm(cm, waves, cmGroups, s), "context modelling");
     if (!capturing_) hipCheck(hipEventRecord(ev_[4], s), "event");
-    hipCheck(launch_sort_blocks(dInfo_, n, dHist_, dPerm_, dCounters_, s), "block ordering");
-    hipCheck(launch_out_offsets(dInfo_, n, dOutOff_, dPartial_, s), "codeword offsets");
+    hipCheck(launch_plan(dInfo_, n, dOrder_, dPerm_, dOutOff_, dPartial_, dCounters_, s), "block order and codeword offsets");
     MqParams mq{};
     mq.info = dInfo_;
     mq.chunks = dChunks_;
@@ -797,7 +796,7 @@ void Job::enqueueT1(hipStream_t s) {
         rp.counters = dCounters_;
         hipCheck(launch_rc(rp, numFrames(), rcMaxBlocks_, rcMaxPackets_, s), "rate control");
     }
-    hipCheck(launch_compact_offsets(dInfo_, dCodeLen_, n, dDataOff_, nullptr, dPartial_, s), "compaction offsets");
+    hipCheck(launch_compact_offsets(dInfo_, dCodeLen_, n, dDataOff_, dPartial_, dCounters_, s), "compaction offsets");
     // dense results live in the (now consumed) symbol pool
     const size_t dataBytes = alignUp(outCap_);
     dDenseData_ = dPool_;
@@ -821,9 +820,7 @@ void Job::enqueueT1(hipStream_t s) {
     hipCheck(launch_compact(cp, s), "compaction");
     if (!capturing_) hipCheck(hipEventRecord(ev_[6], s), "event");
     // flags and totals for finish()
-    const int groups = (int)((n + 2047) / 2048);
     hipCheck(hipMemcpyAsync(hSmall_, dCounters_, sizeof(JobCounters), hipMemcpyDeviceToHost, s), "counters");
-    hipCheck(hipMemcpyAsync(hSmall_ + 16, dPartial_ + groups, 8, hipMemcpyDeviceToHost, s), "totals");
 }
 
 void Job::enqueueChain(bool uploadInputs) {
@@ -939,7 +936,7 @@ void Job::finish(StageTimes* times) {
         enqueueT1(stream_);
         hipCheck(hipStreamSynchronize(stream_), "encode (re-run)");
     }
-    const unsigned long long packed = hSmall_[16];
+    const unsigned long long packed = ((const JobCounters*)hSmall_)->kept;
     numDataTotal_ = (size_t)(packed & ((1ull << 36) - 1));
     numPassesTotal_ = (size_t)(packed >> 36);
     if (numPassesTotal_ > hPassCap_) {

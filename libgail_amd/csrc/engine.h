@@ -309,7 +309,7 @@ private:
     uint2* dChunks_ = nullptr;
     MqSnapshot* dSnaps_ = nullptr;
     uint32_t* dPerm_ = nullptr;
-    uint32_t* dHist_ = nullptr;
+    uint32_t* dOrder_ = nullptr;
     unsigned long long* dOutOff_ = nullptr;
     unsigned long long* dDataOff_ = nullptr;
     unsigned long long* dPartial_ = nullptr;
@@ -331,7 +331,7 @@ private:
     int32_t* hPassDist_ = nullptr;
     uint8_t* hData_ = nullptr;
     size_t hDataCap_ = 0, hPassCap_ = 0;
-    unsigned long long* hSmall_ = nullptr;  // counters + totals
+    unsigned long long* hSmall_ = nullptr;  // the counters
     size_t numPassesTotal_ = 0, numDataTotal_ = 0;
     std::vector<size_t> frameDataBase_, framePassBase_;
 };

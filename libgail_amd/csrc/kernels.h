@@ -139,16 +139,19 @@ hipError_t launch_color(const ColorDesc& d, hipStream_t s);
 
 // Uploads the constant context and probability tables; call once per device before any launch.
 hipError_t t1_tables_init();
-hipError_t launch_clear_counters(JobCounters* c, uint32_t* work, int nwork, hipStream_t s);
+// order: kOrderWords words of the block ordering, cleared here and used by launch_plan.
+constexpr int kOrderWords = 256;
+hipError_t launch_clear_counters(JobCounters* c, uint32_t* work, int nwork, uint32_t* order, hipStream_t s);
 hipError_t launch_t1_cm(const CmParams& p, int waves_per_group, int groups, hipStream_t s);
-hipError_t launch_sort_blocks(const T1Info* info, uint32_t n, uint32_t* hist, uint32_t* perm, JobCounters* counters,
-                              hipStream_t s);
-hipError_t launch_out_offsets(const T1Info* info, uint32_t n, unsigned long long* out_off, unsigned long long* partial,
-                              hipStream_t s);
+// Block order (largest first) and codeword offsets; partial: an entry per group of
+// kPlanGroupBlocks blocks.
+constexpr int kPlanGroupBlocks = 1024;
+hipError_t launch_plan(const T1Info* info, uint32_t n, uint32_t* order, uint32_t* perm, unsigned long long* out_off,
+                       unsigned long long* partial, JobCounters* counters, hipStream_t s);
 // group: lanes per workgroup (64, 128, 256); read_bytes: symbols read per lane at a time (16 or 64).
 hipError_t launch_t1_mq(const MqParams& p, int group, int read_bytes, int groups, hipStream_t s);
 hipError_t launch_compact_offsets(const T1Info* info, const uint32_t* code_len, uint32_t n,
-                                  unsigned long long* data_off, uint32_t* pass_off, unsigned long long* partial,
+                                  unsigned long long* data_off, unsigned long long* partial, JobCounters* counters,
                                   hipStream_t s);
 hipError_t launch_compact(const CompactParams& p, hipStream_t s);
 hipError_t launch_quant_debug(const T1Block* blocks, const T1Band* bands, const T1FrameRef* frames, uint32_t n,

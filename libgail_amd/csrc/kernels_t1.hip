@@ -113,14 +113,16 @@ constexpr int kChunkBytes = 65536;  // symbol pool grabbed per wave at a time
 }  // namespace
 
 // ---------------------------------------------------------------- counters
-__global__ void clear_counters_kernel(JobCounters* c, uint32_t* work, int nwork) {
+__global__ void clear_counters_kernel(JobCounters* c, uint32_t* work, int nwork, uint32_t* order) {
     const int t = threadIdx.x;
     if (t < (int)(sizeof(JobCounters) / 4)) ((uint32_t*)c)[t] = 0;
     if (t < nwork) work[t] = 0;
+    order[t] = 0;
 }
 
-hipError_t launch_clear_counters(JobCounters* c, uint32_t* work, int nwork, hipStream_t s) {
-    hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, s, c, work, nwork);
+hipError_t launch_clear_counters(JobCounters* c, uint32_t* work, int nwork, uint32_t* order, hipStream_t s) {
+    static_assert(sizeof(JobCounters) / 4 <= kOrderWords);
+    hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(kOrderWords), 0, s, c, work, nwork, order);
     return hipGetLastError();
 }
 
@@ -599,13 +601,21 @@ hipError_t launch_t1_cm(const CmParams& p, int waves, int groups, hipStream_t s)
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------- ordering
-// Counting sort of the blocks by symbol count, largest first: 128 buckets, four per
-// octave. Kernel 1 histograms, kernel 2 turns the histogram into bucket starts, kernel 3
-// scatters (one global reservation per bucket and workgroup).
+// ---------------------------------------------------------------- ordering and offsets
+// Before MQ coding: a counting sort of the blocks by symbol count, largest first (128 buckets,
+// four per octave), and the exclusive sum of their codewords' capacities; before compaction: the
+// exclusive sum of what is kept. Each takes two launches over groups of kPlanSpan blocks: the
+// first counts and sums per group, and in the second every group adds up the counts and sums
+// of those before it for itself. These kernels do next to nothing and cost their launch, 4 us and
+// more each, so there are few: with the clearing, the scans of the counts and of the sums and the
+// capacities' own two passes as separate launches, ten in all, these kernels took 59 us of one 4K
+// frame, now 20; of 16 frames 102, now 49.
 namespace {
 constexpr int kBuckets = 128;
-constexpr int kSortSpan = 4096;  // blocks per workgroup
+constexpr int kPlanSpan = kPlanGroupBlocks;  // blocks per workgroup
+constexpr int kPlanPer = kPlanSpan / 256;
+static_assert(kOrderWords == 2 * kBuckets);
+
 __device__ __forceinline__ uint32_t bucket_of(uint32_t s) {
     if (s < 4) return kBuckets - 1;
     const int l = 31 - __clz((int)s);
@@ -613,78 +623,6 @@ __device__ __forceinline__ uint32_t bucket_of(uint32_t s) {
     const uint32_t b = (uint32_t)l * 4 + sub;
     return kBuckets - 1 - (b < kBuckets - 1 ? b : kBuckets - 1);
 }
-}  // namespace
-
-__global__ void __launch_bounds__(256) sort_hist_kernel(const T1Info* info, uint32_t n, uint32_t* hist,
-                                                        JobCounters* counters) {
-    __shared__ uint32_t h[kBuckets];
-    __shared__ unsigned long long total;
-    for (int i = threadIdx.x; i < kBuckets; i += 256) h[i] = 0;
-    if (threadIdx.x == 0) total = 0;
-    __syncthreads();
-    const uint32_t b0 = blockIdx.x * kSortSpan, b1 = min(n, b0 + kSortSpan);
-    unsigned long long mine = 0;
-    for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256) {
-        const uint32_t s = info[i].symbols;
-        mine += s;
-        atomicAdd(&h[bucket_of(s)], 1u);
-    }
-    atomicAdd(&total, mine);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kBuckets; i += 256)
-        if (h[i]) atomicAdd(&hist[i], h[i]);
-    if (threadIdx.x == 0) atomicAdd(&counters->symbols, total);
-}
-
-__global__ void sort_scan_kernel(uint32_t* hist) {
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int b = 0; b < kBuckets; ++b) {
-            const uint32_t c = hist[b];
-            hist[b] = run;
-            run += c;
-        }
-    }
-}
-
-__global__ void __launch_bounds__(256) sort_scatter_kernel(const T1Info* info, uint32_t n, uint32_t* cursor,
-                                                           uint32_t* perm) {
-    __shared__ uint32_t h[kBuckets], base[kBuckets];
-    for (int i = threadIdx.x; i < kBuckets; i += 256) h[i] = 0;
-    __syncthreads();
-    const uint32_t b0 = blockIdx.x * kSortSpan, b1 = min(n, b0 + kSortSpan);
-    for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256) atomicAdd(&h[bucket_of(info[i].symbols)], 1u);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kBuckets; i += 256) {
-        base[i] = h[i] ? atomicAdd(&cursor[i], h[i]) : 0u;
-        h[i] = 0;
-    }
-    __syncthreads();
-    for (uint32_t i = b0 + threadIdx.x; i < b1; i += 256) {
-        const uint32_t b = bucket_of(info[i].symbols);
-        perm[base[b] + atomicAdd(&h[b], 1u)] = i;
-    }
-}
-
-__global__ void zero_u32_kernel(uint32_t* p, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-
-hipError_t launch_sort_blocks(const T1Info* info, uint32_t n, uint32_t* hist, uint32_t* perm, JobCounters* counters,
-                              hipStream_t s) {
-    const uint32_t groups = (n + kSortSpan - 1) / kSortSpan;
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(128), 0, s, hist, kBuckets);
-    hipLaunchKernelGGL(sort_hist_kernel, dim3(groups), dim3(256), 0, s, info, n, hist, counters);
-    hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(64), 0, s, hist);
-    hipLaunchKernelGGL(sort_scatter_kernel, dim3(groups), dim3(256), 0, s, info, n, hist, perm);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- exclusive scans
-// Three-phase exclusive scan over per-block values (kScanSpan blocks per workgroup):
-// per-group totals, a one-group scan of the totals, then local scans plus the group base.
-namespace {
-constexpr int kScanSpan = 2048;
 
 __device__ __forceinline__ uint32_t out_capacity(const T1Info& f) {
     // A block's codeword never needs more than half a byte per symbol plus the flush; a
@@ -692,76 +630,156 @@ __device__ __forceinline__ uint32_t out_capacity(const T1Info& f) {
     return f.passes ? ((f.symbols / 2u + 64u + 63u) & ~63u) : 0u;
 }
 
-template <class F>
-__device__ void block_scan_u64(uint32_t n, unsigned long long* out, unsigned long long* partial, int phase, F value) {
-    __shared__ unsigned long long s[256];
-    const uint32_t b0 = blockIdx.x * kScanSpan, b1 = min(n, b0 + kScanSpan);
-    const uint32_t per = kScanSpan / 256;
-    const uint32_t i0 = b0 + threadIdx.x * per, i1 = min(b1, i0 + per);
-    unsigned long long sum = 0;
-    for (uint32_t i = i0; i < i1; ++i) sum += value(i);
-    s[threadIdx.x] = sum;
+// The sum of v over the 256 threads, in every thread; s holds 4 values.
+__device__ __forceinline__ unsigned long long group_sum(unsigned long long v, unsigned long long* s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-        const unsigned long long v = threadIdx.x >= (unsigned)d ? s[threadIdx.x - d] : 0ull;
-        __syncthreads();
-        s[threadIdx.x] += v;
-        __syncthreads();
+    v = s[0] + s[1] + s[2] + s[3];
+    __syncthreads();
+    return v;
+}
+
+// The sum of v over the threads before this one.
+__device__ __forceinline__ unsigned long long group_before(unsigned long long v, unsigned long long* s) {
+    unsigned long long inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long u = __shfl_up(inc, o);
+        if ((threadIdx.x & 63) >= (unsigned)o) inc += u;
     }
-    if (phase == 0) {
-        if (threadIdx.x == 255) partial[blockIdx.x] = s[255];
-        return;
-    }
-    unsigned long long run = partial[blockIdx.x] + s[threadIdx.x] - sum;
-    for (uint32_t i = i0; i < i1; ++i) {
-        out[i] = run;
-        run += value(i);
-    }
+    if ((threadIdx.x & 63) == 63) s[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    unsigned long long base = 0;
+    for (unsigned k = 0; k < (threadIdx.x >> 6); ++k) base += s[k];
+    __syncthreads();
+    return base + inc - v;
+}
+
+// The sum of the groups' values before group g.
+__device__ __forceinline__ unsigned long long groups_before(const unsigned long long* partial, uint32_t g,
+                                                            unsigned long long* s) {
+    unsigned long long v = 0;
+    for (uint32_t i = threadIdx.x; i < g; i += 256) v += partial[i];
+    return group_sum(v, s);
 }
 }  // namespace
 
-__global__ void __launch_bounds__(256) out_offsets_kernel(const T1Info* info, uint32_t n, unsigned long long* out,
-                                                          unsigned long long* partial, int phase) {
-    block_scan_u64(n, out, partial, phase, [&](uint32_t i) { return (unsigned long long)out_capacity(info[i]); });
-}
-
-__global__ void scan_partials_kernel(unsigned long long* partial, int groups, unsigned long long* total) {
+__global__ void __launch_bounds__(256) plan_count_kernel(const T1Info* info, uint32_t n, uint32_t* order,
+                                                         unsigned long long* partial, JobCounters* counters) {
+    __shared__ uint32_t h[kBuckets];
+    __shared__ unsigned long long s[4];
+    if (threadIdx.x < kBuckets) h[threadIdx.x] = 0;
+    __syncthreads();
+    unsigned long long symbols = 0, bytes = 0;
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        const uint32_t i = blockIdx.x * kPlanSpan + 256 * j + threadIdx.x;
+        if (i >= n) break;
+        const T1Info f = info[i];
+        symbols += f.symbols;
+        bytes += out_capacity(f);
+        atomicAdd(&h[bucket_of(f.symbols)], 1u);
+    }
+    symbols = group_sum(symbols, s);  // its barriers also end the counting
+    bytes = group_sum(bytes, s);
+    if (threadIdx.x < kBuckets && h[threadIdx.x]) atomicAdd(&order[threadIdx.x], h[threadIdx.x]);
     if (threadIdx.x == 0) {
-        unsigned long long run = 0;
-        for (int g = 0; g < groups; ++g) {
-            const unsigned long long c = partial[g];
-            partial[g] = run;
-            run += c;
-        }
-        if (total) *total = run;
+        partial[blockIdx.x] = bytes;
+        atomicAdd(&counters->symbols, symbols);
     }
 }
 
-hipError_t launch_out_offsets(const T1Info* info, uint32_t n, unsigned long long* out_off, unsigned long long* partial,
-                              hipStream_t s) {
-    const int groups = (int)((n + kScanSpan - 1) / kScanSpan);
-    hipLaunchKernelGGL(out_offsets_kernel, dim3(groups), dim3(256), 0, s, info, n, out_off, partial, 0);
-    hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(64), 0, s, partial, groups, partial + groups);
-    hipLaunchKernelGGL(out_offsets_kernel, dim3(groups), dim3(256), 0, s, info, n, out_off, partial, 1);
+__global__ void __launch_bounds__(256) plan_place_kernel(const T1Info* info, uint32_t n, uint32_t* order,
+                                                         const unsigned long long* partial, uint32_t* perm,
+                                                         unsigned long long* out_off) {
+    __shared__ uint32_t h[kBuckets], base[kBuckets];
+    __shared__ unsigned long long s[4];
+    if (threadIdx.x < kBuckets) h[threadIdx.x] = 0;
+    const unsigned long long start = group_before(threadIdx.x < kBuckets ? order[threadIdx.x] : 0u, s);
+    unsigned long long run = groups_before(partial, blockIdx.x, s);
+    const uint32_t i0 = blockIdx.x * kPlanSpan + kPlanPer * threadIdx.x;
+    T1Info f[kPlanPer];
+    unsigned long long bytes = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        f[j] = i0 + j < n ? info[i0 + j] : T1Info{};
+        bytes += out_capacity(f[j]);
+        if (i0 + j < n) atomicAdd(&h[bucket_of(f[j].symbols)], 1u);
+    }
+    run += group_before(bytes, s);
+#pragma unroll
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        if (i0 + j < n) out_off[i0 + j] = run;
+        run += out_capacity(f[j]);
+    }
+    // one reservation per bucket and group, in the bucket's cursor
+    if (threadIdx.x < kBuckets) {
+        base[threadIdx.x] =
+            (uint32_t)start + (h[threadIdx.x] ? atomicAdd(&order[kBuckets + threadIdx.x], h[threadIdx.x]) : 0u);
+        h[threadIdx.x] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < kPlanPer; ++j)
+        if (i0 + j < n) {
+            const uint32_t b = bucket_of(f[j].symbols);
+            perm[base[b] + atomicAdd(&h[b], 1u)] = i0 + j;
+        }
+}
+
+hipError_t launch_plan(const T1Info* info, uint32_t n, uint32_t* order, uint32_t* perm, unsigned long long* out_off,
+                       unsigned long long* partial, JobCounters* counters, hipStream_t s) {
+    const uint32_t groups = (n + kPlanSpan - 1) / kPlanSpan;
+    hipLaunchKernelGGL(plan_count_kernel, dim3(groups), dim3(256), 0, s, info, n, order, partial, counters);
+    hipLaunchKernelGGL(plan_place_kernel, dim3(groups), dim3(256), 0, s, info, n, order, partial, perm, out_off);
     return hipGetLastError();
 }
 
+// What a block keeps: its codeword's bytes in whole words, and its passes << 36.
+__device__ __forceinline__ unsigned long long kept_size(const T1Info* info, const uint32_t* len, uint32_t i) {
+    return (unsigned long long)((len[i] + 3u) & ~3u) | ((unsigned long long)info[i].passes << 36);
+}
+
+__global__ void __launch_bounds__(256) data_sizes_kernel(const T1Info* info, const uint32_t* len, uint32_t n,
+                                                         unsigned long long* partial) {
+    __shared__ unsigned long long s[4];
+    unsigned long long v = 0;
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        const uint32_t i = blockIdx.x * kPlanSpan + 256 * j + threadIdx.x;
+        if (i < n) v += kept_size(info, len, i);
+    }
+    v = group_sum(v, s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = v;
+}
+
 __global__ void __launch_bounds__(256) data_offsets_kernel(const T1Info* info, const uint32_t* len, uint32_t n,
-                                                           unsigned long long* out, unsigned long long* partial,
-                                                           int phase) {
-    block_scan_u64(n, out, partial, phase, [&](uint32_t i) {
-        return (unsigned long long)((len[i] + 3u) & ~3u) | ((unsigned long long)info[i].passes << 36);
-    });
+                                                           const unsigned long long* partial,
+                                                           unsigned long long* data_off, JobCounters* counters) {
+    __shared__ unsigned long long s[4];
+    unsigned long long run = groups_before(partial, blockIdx.x, s);
+    const uint32_t i0 = blockIdx.x * kPlanSpan + kPlanPer * threadIdx.x;
+    unsigned long long v[kPlanPer], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        v[j] = i0 + j < n ? kept_size(info, len, i0 + j) : 0ull;
+        sum += v[j];
+    }
+    run += group_before(sum, s);
+#pragma unroll
+    for (uint32_t j = 0; j < kPlanPer; ++j) {
+        if (i0 + j < n) data_off[i0 + j] = run;
+        run += v[j];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) counters->kept = run;
 }
 
 hipError_t launch_compact_offsets(const T1Info* info, const uint32_t* code_len, uint32_t n,
-                                  unsigned long long* data_off, uint32_t* pass_off, unsigned long long* partial,
+                                  unsigned long long* data_off, unsigned long long* partial, JobCounters* counters,
                                   hipStream_t s) {
-    (void)pass_off;
-    const int groups = (int)((n + kScanSpan - 1) / kScanSpan);
-    hipLaunchKernelGGL(data_offsets_kernel, dim3(groups), dim3(256), 0, s, info, code_len, n, data_off, partial, 0);
-    hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(64), 0, s, partial, groups, partial + groups);
-    hipLaunchKernelGGL(data_offsets_kernel, dim3(groups), dim3(256), 0, s, info, code_len, n, data_off, partial, 1);
+    const uint32_t groups = (n + kPlanSpan - 1) / kPlanSpan;
+    hipLaunchKernelGGL(data_sizes_kernel, dim3(groups), dim3(256), 0, s, info, code_len, n, partial);
+    hipLaunchKernelGGL(data_offsets_kernel, dim3(groups), dim3(256), 0, s, info, code_len, n, partial, data_off, counters);
     return hipGetLastError();
 }
 
