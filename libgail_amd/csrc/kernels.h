@@ -120,7 +120,8 @@ struct RcParams {
 constexpr int kRcDistSums = 1024;
 size_t rc_run_bytes(size_t frames);
 // Entries of RcParams::part for a job of `blocks` code-blocks in `frames` frames.
-inline size_t rcPartEntries(size_t blocks, size_t frames) { return blocks / 256 + frames + 2; }
+constexpr int kRcPartBlocks = 64;  // blocks of a hull workgroup
+inline size_t rcPartEntries(size_t blocks, size_t frames) { return blocks / kRcPartBlocks + frames + 2; }
 size_t rc_segsum_entries(size_t frames);
 hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, uint32_t max_frame_packets,
                      hipStream_t s);

@@ -46,7 +46,8 @@ __device__ __forceinline__ void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int kHullThreads = 256;  // blocks per hull / fill workgroup (one partial slope range each)
+constexpr int kHullGroup = kRcPartBlocks;  // blocks per hull workgroup (one partial slope range each)
+constexpr int kHullThreads = 256;          // blocks per fill workgroup
 constexpr int kScanThreads = 256;
 constexpr int kScanBins = 4 * kScanThreads;  // bins per scan workgroup
 constexpr int kScanSegs = (kRcMaxBins + 1 + kScanBins - 1) / kScanBins;
@@ -62,7 +63,7 @@ __device__ __forceinline__ uint32_t* hist_of(const RcParams& P, uint32_t f, int 
 
 // Partial slope range of hull workgroup x of frame f: frames never share an entry.
 __device__ __forceinline__ uint32_t part_index(const RcFrame& F, uint32_t f, uint32_t x) {
-    return F.first_block / kHullThreads + f + x;
+    return F.first_block / kHullGroup + f + x;
 }
 
 // RcSearch's view of the histogram sums, for a whole wave that runs the search with the same
@@ -88,71 +89,99 @@ struct DevHistView {
     }
 };
 
-// Point-major hull store of one block.
+// Widens a slope range (the bits of positive doubles, ~0 and 0 when empty) by another.
+__device__ __forceinline__ void slope_range(unsigned long long& lo, unsigned long long& hi, unsigned long long lo2,
+                                            unsigned long long hi2) {
+    lo = lo2 < lo ? lo2 : lo;
+    hi = hi2 > hi ? hi2 : hi;
+}
+
+// Point-major hull store of one block, with the points' slope bins and the slope range.
 struct HullSink {
-    double* slope;
-    double* gain;
-    uint32_t* sel;
-    size_t stride;
-    __device__ void operator()(int j, const RcPoint& q) const {
-        const size_t at = (size_t)j * stride;
-        slope[at] = q.slope;
-        gain[at] = q.gain;
-        sel[at] = q.passes << 24 | q.rate;
+    const RcParams& P;
+    uint32_t cb;
+    unsigned long long lmin, lmax;  // positive doubles order as their bits
+    __device__ void operator()(int j, const RcPoint& q) {
+        const size_t at = (size_t)j * P.stride + cb;
+        P.h_slope[at] = q.slope;
+        P.h_gain[at] = q.gain;
+        P.h_sel[at] = q.passes << 24 | q.rate;
+        int32_t k;
+        if (!rc_finite(q.slope)) k = kBinAbove;
+        else if (!(q.slope > 0)) k = kBinBelow;
+        else {
+            k = (int32_t)rc_slope_bin(q.slope, P.mantissa, P.first);
+            const unsigned long long bits = __builtin_bit_cast(unsigned long long, q.slope);
+            lmin = bits < lmin ? bits : lmin;
+            lmax = bits > lmax ? bits : lmax;
+        }
+        P.h_kbin[at] = k;
     }
+};
+
+// A block's pass tables are rows of kMaxPasses entries: four at a time, the last four again
+// beyond the row's end.
+struct DevPassRows {
+    const uint4* len;
+    const int4* dist;
+    __device__ void load(int k, int, uint32_t* l, int32_t* d) const {
+        const int q = min(k >> 2, kMaxPasses / 4 - 1);
+        const uint4 a = len[q];
+        const int4 b = dist[q];
+        l[0] = a.x, l[1] = a.y, l[2] = a.z, l[3] = a.w;
+        d[0] = b.x, d[1] = b.y, d[2] = b.z, d[3] = b.w;
+    }
+};
+
+// The hull under construction, a column of LDS per lane.
+struct DevHullStack {
+    uint32_t (*sel)[64];  // passes << 24 | rate
+    double (*D)[64];
+    int lane;
+    __device__ void put(int m, uint32_t r, uint32_t k, double d) {
+        sel[m][lane] = k << 24 | r;
+        D[m][lane] = d;
+    }
+    __device__ uint32_t rate(int m) const { return sel[m][lane] & 0xFFFFFFu; }
+    __device__ uint32_t passes(int m) const { return sel[m][lane] >> 24; }
+    __device__ double dist(int m) const { return D[m][lane]; }
 };
 
 }  // namespace
 
-__global__ void __launch_bounds__(kHullThreads) rc_hull_kernel(RcParams P) {
-    __shared__ unsigned long long s_min, s_max;
+// Bound by latency (a serial scan of each block's passes with a division or more per pass). The
+// stack is in LDS, 50 KB a wave, so one-wave workgroups, three to a CU: with the stack in
+// scratch memory and the bins from a second pass over the stored slopes one 4K frame took 118 us
+// and 16 frames 404, now 38 and 184.
+__global__ void __launch_bounds__(kHullGroup) rc_hull_kernel(RcParams P) {
+    __shared__ double s_D[kMaxPasses + 1][64];
+    __shared__ uint32_t s_sel[kMaxPasses + 1][64];
+    static_assert(kHullGroup == 64);
     const uint32_t f = blockIdx.y;
     const RcFrame& F = P.frames[f];
     if (F.max_total == 0) return;          // no rate control for this frame
     if (P.counters->flags & 3u) return;    // Tier-1 overflowed: the job is re-run
-    if (blockIdx.x * kHullThreads >= F.nblocks) return;
-    const int t = threadIdx.x;
-    if (t == 0) {
-        s_min = ~0ull;
-        s_max = 0ull;
-    }
-    __syncthreads();
-    const uint32_t i = blockIdx.x * kHullThreads + t;
+    if (blockIdx.x * kHullGroup >= F.nblocks) return;
+    const uint32_t i = blockIdx.x * kHullGroup + threadIdx.x;
     unsigned long long lmin = ~0ull, lmax = 0ull;
     if (i < F.nblocks) {
         const uint32_t cb = F.first_block + i;
         const T1Info inf = P.info[cb];
-        const int np = (int)inf.passes;
         const uint32_t band = P.blocks[cb].band;
-        const int cnt = np ? rc_block_hull_to(np, (int)inf.nbps, P.band_scale[band], P.pass_len + (size_t)cb * kMaxPasses,
-                                              P.pass_dist + (size_t)cb * kMaxPasses,
-                                              HullSink{P.h_slope + cb, P.h_gain + cb, P.h_sel + cb, P.stride})
-                           : 0;
+        DevHullStack stack{s_sel, s_D, (int)threadIdx.x};
+        HullSink sink{P, cb, lmin, lmax};
+        const DevPassRows rows{(const uint4*)(P.pass_len + (size_t)cb * kMaxPasses),
+                               (const int4*)(P.pass_dist + (size_t)cb * kMaxPasses)};
+        const int cnt = rc_block_hull_to((int)inf.passes, (int)inf.nbps, P.band_scale[band], rows, stack, sink);
         P.hull_n[cb] = (uint32_t)cnt | (P.bands[band].comp_mb & 3u) << 8;
-        for (int h = 0; h < cnt; ++h) {
-            const size_t at = (size_t)h * P.stride + cb;
-            const double s = P.h_slope[at];
-            int32_t k;
-            if (!rc_finite(s)) k = kBinAbove;
-            else if (!(s > 0)) k = kBinBelow;
-            else {
-                k = (int32_t)rc_slope_bin(s, P.mantissa, P.first);
-                const unsigned long long bits = __builtin_bit_cast(unsigned long long, s);  // positive doubles order as their bits
-                lmin = bits < lmin ? bits : lmin;
-                lmax = bits > lmax ? bits : lmax;
-            }
-            P.h_kbin[at] = k;
-        }
+        lmin = sink.lmin;
+        lmax = sink.lmax;
     }
-    if (lmax) {
-        atomicMin(&s_min, lmin);
-        atomicMax(&s_max, lmax);
-    }
-    __syncthreads();
-    if (t == 0) {
+    for (int o = 32; o > 0; o >>= 1) slope_range(lmin, lmax, __shfl_xor(lmin, o), __shfl_xor(lmax, o));
+    if (threadIdx.x == 0) {
         unsigned long long* part = P.part + 2 * (size_t)part_index(F, f, blockIdx.x);
-        part[0] = s_min;
-        part[1] = s_max;
+        part[0] = lmin;
+        part[1] = lmax;
     }
 }
 
@@ -168,13 +197,16 @@ __global__ void __launch_bounds__(kHullThreads) rc_range_kernel(RcParams P) {
         s_max = 0ull;
     }
     __syncthreads();
-    const uint32_t nparts = (F.nblocks + kHullThreads - 1) / kHullThreads;
+    const uint32_t nparts = (F.nblocks + kHullGroup - 1) / kHullGroup;
+    unsigned long long lmin = ~0ull, lmax = 0ull;
     for (uint32_t x = t; x < nparts; x += kHullThreads) {
         const unsigned long long* part = P.part + 2 * (size_t)part_index(F, f, x);
-        if (part[1]) {
-            atomicMin(&s_min, part[0]);
-            atomicMax(&s_max, part[1]);
-        }
+        slope_range(lmin, lmax, part[0], part[1]);
+    }
+    for (int o = 32; o > 0; o >>= 1) slope_range(lmin, lmax, __shfl_xor(lmin, o), __shfl_xor(lmax, o));
+    if ((t & 63) == 0) {
+        atomicMin(&s_min, lmin);
+        atomicMax(&s_max, lmax);
     }
     __syncthreads();
     if (t == 0) {
@@ -643,7 +675,8 @@ hipError_t launch_rc(const RcParams& p, int frames, uint32_t max_frame_blocks, u
                      hipStream_t s) {
     const uint32_t gx = (max_frame_blocks + kHullThreads - 1) / kHullThreads;
     if (!gx || !frames) return hipSuccess;
-    hipLaunchKernelGGL(rc_hull_kernel, dim3(gx, frames), dim3(kHullThreads), 0, s, p);
+    const uint32_t hx = (max_frame_blocks + kHullGroup - 1) / kHullGroup;
+    hipLaunchKernelGGL(rc_hull_kernel, dim3(hx, frames), dim3(kHullGroup), 0, s, p);
     hipLaunchKernelGGL(rc_range_kernel, dim3(frames), dim3(kHullThreads), 0, s, p);
     hipLaunchKernelGGL(rc_fill_kernel, dim3(gx, frames), dim3(kHullThreads), 0, s, p);
     hipLaunchKernelGGL(rc_scan_kernel<0>, dim3(kScanSegs, 6, frames), dim3(kScanThreads), 0, s, p);

@@ -28,43 +28,66 @@ GAIL_HD double rc_plane_scale(int nbps, int k) {
     return (double)(1ull << (2 * plane)) / 4096.0;
 }
 
-// Lower convex hull of a block's (rate, distortion) points (rate_control.cpp:38-86): len and
-// dist are the block's cumulative truncation lengths and per-pass distortion reductions,
-// scale is delta^2 * weight of its subband. Hands point j to out(j, point) and returns the
-// number of points; their slopes fall strictly (the first may be infinite).
-template <class Sink>
-GAIL_HD int rc_block_hull_to(int np, int nbps, double scale, const uint32_t* len, const int32_t* dist, const Sink& out) {
-    uint32_t R[kMaxPasses + 1];
-    double D[kMaxPasses + 1];
-    int K[kMaxPasses + 1];
+// Lower convex hull of a block's (rate, distortion) points (rate_control.cpp:38-86): pass
+// gives its cumulative truncation lengths and per-pass distortion reductions four passes at a
+// time, scale is delta^2 * weight of its subband, stack keeps the hull's points (rate, passes
+// and distortion, 0 the origin) while it is built. Hands point j to out(j, point) and returns
+// the number of points; their slopes fall strictly (the first may be infinite).
+template <class Passes, class Stack, class Sink>
+GAIL_HD int rc_block_hull_to(int np, int nbps, double scale, const Passes& pass, Stack& stack, Sink& out) {
     int m = 0;
-    R[0] = 0;
-    D[0] = 0.0;
-    K[0] = 0;
+    uint32_t R = 0;          // the hull's last point
+    double D = 0, last = 0;  // and the slope that leads to it (m > 0)
+    stack.put(0, 0, 0, 0.0);
     double acc = 0;
-    for (int k = 0; k < np; ++k) {
-        acc += (double)dist[k] * rc_plane_scale(nbps, k) * scale;
-        const uint32_t r = len[k];
-        if (acc <= D[m]) continue;
-        while (m >= 1) {
-            const double sNew = r == R[m] ? rc_inf() : (acc - D[m]) / (double)(r - R[m]);
-            const double sLast = R[m] == R[m - 1] ? rc_inf() : (D[m] - D[m - 1]) / (double)(R[m] - R[m - 1]);
-            if (sNew < sLast) break;
-            --m;
+    uint32_t len[4], nextLen[4];
+    int32_t dist[4], nextDist[4];
+    pass.load(0, np, nextLen, nextDist);
+    for (int k0 = 0; k0 < np; k0 += 4) {
+        for (int j = 0; j < 4; ++j) {
+            len[j] = nextLen[j];
+            dist[j] = nextDist[j];
         }
-        ++m;
-        R[m] = r;
-        D[m] = acc;
-        K[m] = k + 1;
+        pass.load(k0 + 4, np, nextLen, nextDist);
+GAIL_UNROLL
+        for (int j = 0; j < 4; ++j) {
+            const int k = k0 + j;
+            if (k >= np) break;
+            acc += (double)dist[j] * rc_plane_scale(nbps, k) * scale;
+            const uint32_t r = len[j];
+            if (acc <= D) continue;
+            double s;
+            for (;;) {
+                s = r == R ? rc_inf() : (acc - D) / (double)(r - R);
+                if (m == 0 || s < last) break;
+                --m;
+                R = stack.rate(m);
+                D = stack.dist(m);
+                if (m) {
+                    const uint32_t R1 = stack.rate(m - 1);
+                    last = R == R1 ? rc_inf() : (D - stack.dist(m - 1)) / (double)(R - R1);
+                }
+            }
+            ++m;
+            R = r;
+            D = acc;
+            last = s;
+            stack.put(m, r, (uint32_t)(k + 1), acc);
+        }
     }
+    uint32_t R0 = 0;
+    double D0 = 0;
     for (int j = 1; j <= m; ++j) {
-        const double dr = (double)R[j] - (double)R[j - 1];
+        const uint32_t R1 = stack.rate(j);
+        const double D1 = stack.dist(j), dr = (double)R1 - (double)R0;
         RcPoint q;
-        q.slope = dr <= 0 ? rc_inf() : (D[j] - D[j - 1]) / dr;
-        q.gain = D[j] - D[j - 1];
-        q.rate = R[j];
-        q.passes = (uint32_t)K[j];
+        q.gain = D1 - D0;
+        q.slope = dr <= 0 ? rc_inf() : q.gain / dr;
+        q.rate = R1;
+        q.passes = stack.passes(j);
         out(j - 1, q);
+        R0 = R1;
+        D0 = D1;
     }
     return m;
 }
@@ -73,9 +96,33 @@ struct RcPointArray {
     RcPoint* p;
     GAIL_HD void operator()(int j, const RcPoint& q) const { p[j] = q; }
 };
+struct RcPassRows {
+    const uint32_t* len;
+    const int32_t* dist;
+    GAIL_HD void load(int k, int np, uint32_t* l, int32_t* d) const {
+        for (int j = 0; j < 4 && k + j < np; ++j) {
+            l[j] = len[k + j];
+            d[j] = dist[k + j];
+        }
+    }
+};
+struct RcHullStack {
+    uint32_t R[kMaxPasses + 1], K[kMaxPasses + 1];
+    double D[kMaxPasses + 1];
+    GAIL_HD void put(int m, uint32_t r, uint32_t k, double d) {
+        R[m] = r;
+        K[m] = k;
+        D[m] = d;
+    }
+    GAIL_HD uint32_t rate(int m) const { return R[m]; }
+    GAIL_HD uint32_t passes(int m) const { return K[m]; }
+    GAIL_HD double dist(int m) const { return D[m]; }
+};
 
 GAIL_HD int rc_block_hull(int np, int nbps, double scale, const uint32_t* len, const int32_t* dist, RcPoint* out) {
-    return rc_block_hull_to(np, nbps, scale, len, dist, RcPointArray{out});
+    RcHullStack stack;
+    RcPointArray sink{out};
+    return rc_block_hull_to(np, nbps, scale, RcPassRows{len, dist}, stack, sink);
 }
 
 // Passes of a block kept at threshold lambda: up to its last hull point of slope >= lambda.
