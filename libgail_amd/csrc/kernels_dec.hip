@@ -55,8 +55,9 @@ __device__ __forceinline__ bool block_fields(const T1DecodeParams& P, const DecB
 // chain. 4K at 250 Mbit/s (longest block 1,464 bytes, about 12,300 decisions): 2.02 ms, of which a
 // refinement decision takes 280 cycles, another 380, and a sample turning significant about 850
 // more (its sign, the stripe's contexts again). One lane per block, or a wave on the same
-// sequential code with its state in scalar registers for the longest blocks, took 3.87 ms; eight
-// decoders at once 544 frames/s, now 605. With every decision in vector registers it is 2.6 ms
+// sequential code with its state in scalar registers for the longest blocks, took 3.87 ms. The
+// price is throughput: eight decoders at once, everything in HBM, ran 733 frames/s with the lane
+// code and run 634 with a wave per block. With every decision in vector registers it is 2.6 ms
 // (a decision that may end the walk pays 28 cycles and more to get from a vector comparison to
 // a branch), with every one in scalar registers 2.35.
 __global__ void __launch_bounds__(64 * kDecWaves) t1_decode_kernel(T1DecodeParams P) {
