@@ -3,6 +3,9 @@ that are mostly 0xFF, 0x80-0x8F after it (added to the bits before them only whe
 used), markers in mid-codeword, runs of zeros; codewords of 0 to 700 bytes, so that some end in
 the first decisions and some take several windows; 1 to 30 bit-planes; any number of passes;
 blocks of every width and height at the frame's edges. Every word is exact."""
+import json
+import os
+
 import numpy as np
 import pytest
 
@@ -45,3 +48,27 @@ def test_wave_decoder_edges(device, oracle, w, h, fourk, kind):
     bad = int(np.count_nonzero(wav.view(np.uint32) != want_wav.view(np.uint32)))
     assert bad == 0, f"{bad} coefficients differ"
     assert np.array_equal(got, want)
+
+
+def test_overlapping_byte_waits_for_its_shift(device, oracle):
+    """Codewords with a byte of 0x80-0x8F after 0xFF that falls due in a refinement pass when its
+    carry into the upper half of the code register would turn a decision, if it were added before
+    the shift that needs it."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "t1_overlap_blocks.json")
+    with open(path) as f:
+        blocks = json.load(f)
+    layout = g.FrameLayout(64, 64, 0)
+    orient = np.array([layout.bands[b].orient for b in layout.cblks[:, 0]])
+    dec = g.Decoder(device, layout, 0, True)
+    try:
+        for b in blocks:
+            data = np.frombuffer(bytes.fromhex(b["data"]), np.uint8)
+            at = np.flatnonzero((orient == b["orient"]) & (layout.cblks[:, 3] == b["w"]) & (layout.cblks[:, 4] == b["h"]))
+            codes = np.zeros(layout.num_cblks, g.CBLK_CODE)
+            codes[at[0]] = (0, len(data), b["passes"], b["nbps"], 0)
+            got, _, wav = dec.decode(data, codes, wavelet=True)
+            want, want_wav = oracle.decode_frame(64, 64, 0, data, codes, 0, True, want_wavelet=True)
+            assert np.array_equal(wav.view(np.uint32), want_wav.view(np.uint32)), b["data"]
+            assert np.array_equal(got, want), b["data"]
+    finally:
+        dec.close()
