@@ -51,15 +51,18 @@ __device__ __forceinline__ bool block_fields(const T1DecodeParams& P, const DecB
     return d.dst < P.nwords && P.nwords - d.dst >= (h - 1u) * P.stride + w;
 }
 
-// Latency bound: a frame takes as long as its longest block, whose decisions are one serial
-// chain. 4K at 250 Mbit/s (longest block 1,464 bytes, about 12,300 decisions): 2.02 ms, of which a
-// refinement decision takes 280 cycles, another 380, and a sample turning significant about 850
-// more (its sign, the stripe's contexts again). One lane per block, or a wave on the same
-// sequential code with its state in scalar registers for the longest blocks, took 3.87 ms. The
-// price is throughput: eight decoders at once, everything in HBM, ran 733 frames/s with the lane
-// code and run 634 with a wave per block. With every decision in vector registers it is 2.6 ms
-// (a decision that may end the walk pays 28 cycles and more to get from a vector comparison to
-// a branch), with every one in scalar registers 2.35.
+// One frame at a time is bound by latency: it takes as long as its longest block, whose decisions
+// are one serial chain. 4K at 250 Mbit/s: 2.00 ms, its longest block (1,477 bytes) alone 1.92. One
+// lane per block, or a wave on the same sequential code with its state in scalar registers for
+// the longest blocks, took 3.83 ms. With every decision in vector registers it is 2.6 ms (a
+// decision that may end the walk pays 28 cycles and more to get from a vector comparison to a
+// branch).
+//
+// Several decoders at once are bound by scalar issue, one instruction a cycle and CU: 5.3e8 of
+// them in a 4K frame (19 million decisions), 0.87 ms, and 4.4e8 vector instructions beside them.
+// So decode() and the column walk are written for few scalar instructions (t1_wave_mq.h). Eight
+// decoders with everything in HBM run 765-775 frames/s; with 6.5e8 it was 675-690, and with a lane
+// per block 735-750.
 __global__ void __launch_bounds__(64 * kDecWaves) t1_decode_kernel(T1DecodeParams P) {
     __shared__ DecWave s_wave[kDecWaves];
     __shared__ uint2 s_next[kMqCoderStates];
@@ -79,7 +82,6 @@ __global__ void __launch_bounds__(64 * kDecWaves) t1_decode_kernel(T1DecodeParam
     for (int i = t; i < 256; i += 64 * kDecWaves) s_sign[i] = kDecSign[i];
     const uint32_t lane = (uint32_t)t & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    if (lane == 0u) s_wave[wave].ctx[0] = 0u;
     __syncthreads();
     const uint32_t gw = blockIdx.x * kDecWaves + wave;
     if (gw >= P.nblocks) return;
@@ -89,10 +91,11 @@ __global__ void __launch_bounds__(64 * kDecWaves) t1_decode_kernel(T1DecodeParam
     WaveMq mq;
     const uint32_t row = min(lane, 46u);
     mq.next_m = s_next[2u * row].x;
-    mq.next_l = s_next[2u * row].y;
+    mq.next_x = s_next[2u * row].x ^ s_next[2u * row].y;
     mq.next = s_next;
     // contexts start in their Table D.7 states
-    mq.ctx = kDecInitial[lane == 0u ? 1u : (lane == 17u ? 2u : (lane == 18u ? 3u : 0u))];
+    mq.ctx = kDecInitial[lane == 1u ? 1u : (lane == 18u ? 2u : (lane == 19u ? 3u : 0u))];
+    mq.ctx = lane == 0u ? 0u : mq.ctx;
     mq.ws = &s_wave[wave];
     mq.src = P.bytes + d.off;
     mq.len = d.len;

@@ -26,7 +26,7 @@
 
 namespace gail_amd {
 
-constexpr uint32_t kDecRun = 18u << 2;  // a column in run-length mode
+constexpr uint32_t kDecRun = (17u + 1u) << 2;  // a column in run-length mode
 
 // Inclusive prefix sum over each half-wave.
 __device__ __forceinline__ uint32_t dw_scan(uint32_t v) {
@@ -118,20 +118,23 @@ __device__ __forceinline__ void t1_decode_wave(WaveMq& mq, uint32_t w, uint32_t 
                 word = __builtin_amdgcn_perm(0u, ((word + 0x01010101u) << 2) | 0x03020100u, pack[todo]);
                 word = run ? kDecRun : word;
                 uint32_t cols = (uint32_t)__builtin_amdgcn_ballot_w64(todo != 0u);
-                uint32_t c = 0, pk = 0, was = 0, one = 0;
+                // Both loops end on a value that the decision's bit 31 is part of: with a flag and
+                // jumps out of them the compiler keeps conditions in register pairs, a third more
+                // scalar instructions.
+                uint32_t c = 0, pk = 0, was = 0, d = 0;
                 if (cols) do {
                     c = (uint32_t)__builtin_ctz(cols);
                     pk = dw_lane(word, c);
                     do {
                         was = pk;
-                        one = mq.decode(((pk >> 2) & 31u) - 1u);
-                        pk = (pk >> 8) | (one << 31);  // a sample turned significant: the loops end
+                        d = mq.decode(pk >> 2);
+                        pk = (pk >> 8) | (d & 0x80000000u);  // a sample turned significant: the loops end
                         asm("" : "+s"(pk));
                     } while ((int32_t)pk > 0);
-                    cols = one ? 0u : cols & (cols - 1u);
+                    cols &= (cols - 1u) & ~(uint32_t)((int32_t)d >> 31);
                     asm("" : "+s"(cols));
                 } while (cols);
-                if (!one) {
+                if ((int32_t)d >= 0) {
                     if (type == 0u) V |= todo << r0;
                     break;
                 }
@@ -143,7 +146,7 @@ __device__ __forceinline__ void t1_decode_wave(WaveMq& mq, uint32_t w, uint32_t 
                 if (i == 0u) k = 0u;
                 uint32_t flip = 0, neg;
                 for (;;) {
-                    uint32_t cx = 18u;
+                    uint32_t cx = 18u + 1u;
                     if (i == 2u) {
                         auto side = [](uint32_t s, uint32_t g, uint32_t row) {
                             return ((s >> row) & 1u) | (((g >> row) & 1u) << 1);
@@ -153,9 +156,9 @@ __device__ __forceinline__ void t1_decode_wave(WaveMq& mq, uint32_t w, uint32_t 
                                                 (side(S << 1, G << 1, row) << 4) | (side(S >> 1, G >> 1, row) << 6);
                         const uint32_t sc = dw_lane(sign_lut[around], c);
                         flip = sc & 1u;
-                        cx = (sc >> 1) - 1u;
+                        cx = sc >> 1;
                     }
-                    const uint32_t d = mq.decode(cx);
+                    const uint32_t d = mq.decode(cx) >> 31;
                     neg = d ^ flip;
                     if (i == 2u) break;
                     k = (k << 1) | d;

@@ -24,6 +24,10 @@ constexpr int kDecMaxPlanes = 30;
 using DwLanes = uint32_t;  // a value per lane
 using DwPair = uint2;
 DW_FN uint32_t dw_lane(DwLanes v, uint32_t lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane); }
+// lane's value of a ^ (b & mask)
+DW_FN uint32_t dw_lane_masked(DwLanes a, DwLanes b, uint32_t lane, uint32_t mask) {
+    return dw_lane(a ^ (b & mask), lane);
+}
 DW_FN uint32_t dw_uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 DW_FN bool dw_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 DW_FN void dw_set_lane(DwLanes& v, uint32_t lane, uint32_t x) { v = (threadIdx.x & 63u) == lane ? x : v; }
@@ -37,6 +41,9 @@ struct DwPair {
     uint32_t x, y;
 };
 DW_FN uint32_t dw_lane(const DwLanes& v, uint32_t lane) { return v.v[lane]; }
+DW_FN uint32_t dw_lane_masked(const DwLanes& a, const DwLanes& b, uint32_t lane, uint32_t mask) {
+    return a.v[lane] ^ (b.v[lane] & mask);
+}
 DW_FN uint32_t dw_uniform(uint32_t v) { return v; }
 DW_FN bool dw_any(bool c) { return c; }
 DW_FN void dw_set_lane(DwLanes& v, uint32_t lane, uint32_t x) { v.v[lane] = x; }
@@ -69,8 +76,8 @@ struct WaveMq {
     uint32_t hi, lo;  // C
     uint32_t A;       // interval << 15
     int32_t extra;
-    DwLanes ctx;      // lane k: state of context k
-    DwLanes next_m, next_l;  // lane i: the successors of row i with MPS 0
+    DwLanes ctx;      // lane k + 1: state of context k
+    DwLanes next_m, next_x;  // lane i: row i's successor after an MPS, and what differs after an LPS (MPS 0)
     const DwPair* next;       // successors of a state, after an MPS and after an LPS (LDS)
     DecWave* ws;
     const uint8_t* src;
@@ -192,23 +199,25 @@ struct WaveMq {
         return x < y ? 0xFFFFFFFFu : 0u;
 #endif
     }
-    // DECODE (C.3.2) in scalar registers
-    DW_FN uint32_t decode(uint32_t cx) {
-        const uint32_t st = dw_lane(ctx, cx);
+    // DECODE (C.3.2) in scalar registers; at: the lane of the context's state (modulo 64). The
+    // decision is bit 31 of the result. Few scalar instructions are what counts here, 8 without
+    // and 25 with renormalisation: C is the smaller of hi and hi - Qe (which wraps around where
+    // hi < Qe); the comparison is one select where it is used at once and masks made again for
+    // the renormalisation; the choice of the successor is a vector operation.
+    DW_FN uint32_t decode(uint32_t at) {
+        const uint32_t st = dw_lane(ctx, at & 63u);
         const uint32_t qe = st & 0x3FFF8000u;
-        const uint32_t a = A - qe;
-        const uint32_t lower = below(hi, qe);
-        hi -= qe & ~lower;
-        A = a ^ ((a ^ qe) & lower);
-        uint32_t d = st >> 31;
+        const uint32_t a = A - qe, was = hi;
+        const bool lower = hi < qe;
+        hi = lower ? hi : hi - qe;
+        A = lower ? qe : a;
+        uint32_t d = st;
         if (A < 0x40000000u) {  // else the MPS without renormalisation
             // upper sub-interval: the MPS unless a < Qe; lower: the LPS unless a < Qe
-            const uint32_t lps = below(a, qe) ^ lower;
+            const uint32_t lps = below(a, qe) ^ below(was, qe);
             const uint32_t row = (st >> 4) & 63u;
-            const uint32_t m = dw_lane(next_m, row), l = dw_lane(next_l, row);
-            const uint32_t to = m ^ ((m ^ l) & lps) ^ (st & 0x80000008u);
-            dw_set_lane(ctx, cx, to);
-            d ^= lps & 1u;
+            dw_set_lane(ctx, at & 63u, dw_lane_masked(next_m, next_x, row, lps) ^ (st & 0x80000008u));
+            d ^= lps;
             uint32_t n = (uint32_t)__builtin_clz(A) - 1u;
             A <<= n;
             while (extra < (int32_t)n) {
@@ -231,7 +240,7 @@ struct WaveMq {
     }
     DW_FN void to_vector() {
         dw_each(ctx, [&](uint32_t lane, uint32_t state) {
-            if (lane < 19u) ws->ctx[lane + 1u] = state;
+            if (lane < 20u) ws->ctx[lane] = state;
         });
         vector();
     }
@@ -241,7 +250,7 @@ struct WaveMq {
         vector();
     }
     DW_FN void to_scalar() {
-        dw_each(ctx, [&](uint32_t lane, uint32_t& state) { state = ws->ctx[lane < 19u ? lane + 1u : 0u]; });
+        dw_each(ctx, [&](uint32_t lane, uint32_t& state) { state = ws->ctx[lane < 20u ? lane : 0u]; });
         scalar();
     }
     DW_FN void scalar() {
@@ -335,7 +344,7 @@ DW_UNROLL
                     got = 0u;
                     for (uint32_t j = 0; j < 4u; ++j) {
                         const uint32_t s = (w >> (8u * j + 2u)) & 31u;
-                        if (s) got |= decode(s - 1u) << j;
+                        if (s) got |= (decode(s) >> 31) << j;
                     }
                     to_vector();
                     f.state = *slot(w1);

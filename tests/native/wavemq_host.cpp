@@ -48,8 +48,8 @@ struct Wave {
         for (uint32_t lane = 0; lane < 64; ++lane) {
             const uint32_t row = lane < 46 ? lane : 46;
             mq.next_m.v[lane] = g_tab.next[2 * row].x;
-            mq.next_l.v[lane] = g_tab.next[2 * row].y;
-            mq.ctx.v[lane] = g_tab.initial[lane == 0 ? 1 : (lane == 17 ? 2 : (lane == 18 ? 3 : 0))];
+            mq.next_x.v[lane] = g_tab.next[2 * row].x ^ g_tab.next[2 * row].y;
+            mq.ctx.v[lane] = lane ? g_tab.initial[lane == 1 ? 1 : (lane == 18 ? 2 : (lane == 19 ? 3 : 0))] : 0u;
         }
         mq.next = g_tab.next;
         mq.ws = ws.get();
@@ -57,6 +57,7 @@ struct Wave {
         mq.len = len;
         mq.init();
     }
+    uint32_t decide(uint32_t cx) { return mq.decode(cx + 1) >> 31; }
     // Decisions in the given contexts through a stripe's list.
     std::vector<uint32_t> list(const std::vector<uint32_t>& cx) {
         uint8_t* const l = (uint8_t*)ws->list;
@@ -101,7 +102,7 @@ int host_wave_t1_words(const uint8_t* data, uint32_t len, int w, int h, int orie
     auto significant = [&](int y, int x) {
         auto side = [&](int dy, int dx) { return sig[y + 1 + dy][x + 1 + dx] | neg[y + 1 + dy][x + 1 + dx] << 1; };
         const int e = g_tab.sign[side(0, -1) | side(0, 1) << 2 | side(-1, 0) << 4 | side(1, 0) << 6];
-        const uint32_t s = wave.mq.decode((uint32_t)(e >> 1) - 1u) ^ (uint32_t)(e & 1);
+        const uint32_t s = wave.decide((uint32_t)(e >> 1) - 1u) ^ (uint32_t)(e & 1);
         sig[y + 1][x + 1] = 1;
         neg[y + 1][x + 1] = (uint8_t)s;
         words[y * w + x] = (s << 31) | (3u << p);
@@ -131,9 +132,9 @@ int host_wave_t1_words(const uint8_t* data, uint32_t len, int w, int h, int orie
                     bool run = true;
                     for (int k = y0; k < y1; ++k) run = run && !sig[k + 1][x + 1] && !seen[k + 1][x + 1] && !code(k, x);
                     if (run) {
-                        if (!wave.mq.decode(17u)) continue;
-                        y = (int)(wave.mq.decode(18u) << 1);
-                        y = y0 + (y | (int)wave.mq.decode(18u));
+                        if (!wave.decide(17u)) continue;
+                        y = (int)(wave.decide(18u) << 1);
+                        y = y0 + (y | (int)wave.decide(18u));
                         significant(y++, x);
                     }
                 }
@@ -142,7 +143,7 @@ int host_wave_t1_words(const uint8_t* data, uint32_t len, int w, int h, int orie
                     const int c = code(y, x);
                     if (type == 0 && !c) continue;
                     if (type == 0) seen[y + 1][x + 1] = 1;
-                    if (wave.mq.decode(zc[c])) significant(y, x);
+                    if (wave.decide(zc[c])) significant(y, x);
                 }
             }
         }
@@ -190,7 +191,7 @@ int host_wave_mq_fuzz(uint32_t seed, int codewords) {
             for (uint32_t i = 0; i < n; ++i) cx[i] = lists && below(8) ? 14 + below(3) : below(19);
             if (lists) got = wave.list(cx);
             else
-                for (uint32_t i = 0; i < n; ++i) got[i] = wave.mq.decode(cx[i]);
+                for (uint32_t i = 0; i < n; ++i) got[i] = wave.decide(cx[i]);
             for (uint32_t i = 0; i < n; ++i) same = seq.decode(st, cx[i]) == got[i] && same;
             done += n;
         }
