@@ -100,9 +100,9 @@ struct RcPassRows {
     const uint32_t* len;
     const int32_t* dist;
     GAIL_HD void load(int k, int np, uint32_t* l, int32_t* d) const {
-        for (int j = 0; j < 4 && k + j < np; ++j) {
-            l[j] = len[k + j];
-            d[j] = dist[k + j];
+        for (int j = 0; j < 4; ++j) {  // the caller copies all four, also past the last pass
+            l[j] = k + j < np ? len[k + j] : 0u;
+            d[j] = k + j < np ? dist[k + j] : 0;
         }
     }
 };
