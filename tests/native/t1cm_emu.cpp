@@ -22,7 +22,7 @@
 #include <vector>
 
 #include "t1_cm_masks.h"
-#include "t1_tables.h"
+#include "zc_table.h"
 
 using namespace gail_amd;
 
