@@ -332,7 +332,7 @@ GAIL_API int64_t gail_encode_codestream(int width, int height, int fourk, double
                                         const uint32_t* pass_len, const int32_t* pass_dist, const uint8_t* data,
                                         uint64_t num_blocks, double fps, double mbps, uint8_t* out, uint64_t cap,
                                         double* lambda, double* mse, const char* tag);
-/* Frame sizes from buildCodestream and from the device's packet-size code (run on the host)
+/* Frame sizes from buildCodestream and from the lambda search's packet sizes (rc_packet_bytes)
  * over `trials` pass choices; the number of choices where they differ, -1 on error. */
 GAIL_API int gail_rc_measure_check(int width, int height, int fourk, double base_step, const uint32_t* info5,
                                    const uint32_t* pass_len, const int32_t* pass_dist, const uint8_t* data,

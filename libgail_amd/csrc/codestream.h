@@ -86,8 +86,8 @@ struct RcTables {
     unsigned long long fixedBytes = 0;  // main header, COM reserve, EOC
 };
 RcTables makeRcTables(const Layout& L);
-// Codestream sizes from the tables and rc_packet_bytes (what the device computes) for
-// passes[i] passes of block i.
+// Codestream sizes from the tables and rc_packet_bytes for passes[i] passes of block i: what the
+// device's measurements (kernels_rc.hip) must come to.
 CodestreamSizes rcMeasure(const Layout& L, const RcTables& T, const Tier1Ref& t1, const uint8_t* passes);
 
 // PCRD-opt under the limits (rate_control.cpp:165-279).

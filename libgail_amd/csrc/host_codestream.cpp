@@ -59,8 +59,8 @@ extern "C" GAIL_AMD_EXPORT int64_t gail_encode_codestream(int W, int H, int four
     }
 }
 
-// Sizes of the same frame measured two ways, buildCodestream and the device's packet-size
-// code run on the host, over `trials` pass choices (all passes, none, and random truncations
+// Sizes of the same frame measured two ways, buildCodestream and the packet sizes of the lambda
+// search (rc_packet_bytes), over `trials` pass choices (all passes, none, and random truncations
 // from seed); returns the number of choices where any size differs, or -1 on error.
 extern "C" GAIL_AMD_EXPORT int gail_rc_measure_check(int W, int H, int fourk, double baseStep, const uint32_t* info5,
                                                      const uint32_t* passLen, const int32_t* passDist,

@@ -328,9 +328,12 @@ __global__ void __launch_bounds__(kScanThreads) rc_scan_kernel(RcParams P) {
 
 namespace {
 
-// Waits for an atomic that returned v: what the device-scope atomics of a workgroup's other waves
-// and of later ones read is then in place, without the write-back of the whole L2 that a
-// device-scope fence costs (a measurement of 16 4K frames 285 us with fences, 50 without).
+// Waits for an atomic that returned v, so that a ticket taken afterwards (RcRun::arrived, summed)
+// tells the last workgroup that the value is in place. There is no release and no acquire: a
+// device-scope fence writes back the whole L2 (a measurement of 16 4K frames 285 us with fences,
+// 50 without). So only what is written by device-scope atomics and read by them, past the L2s
+// that the XCDs have of their own, may cross to the last workgroup of the same launch. A plain
+// store (a block's choice, its length) is seen by the next launch, not by that workgroup.
 __device__ __forceinline__ void atomic_done(unsigned long long v) {
     asm volatile("" ::"v"((uint32_t)v), "v"((uint32_t)(v >> 32)) : "memory");
 }
@@ -563,7 +566,8 @@ __global__ void __launch_bounds__(kMeasureWaves * 64) rc_measure_kernel(RcParams
         const unsigned long long b = measure_packet(P, F, k, lambda, s_words[wv]);
         if ((threadIdx.x & 63) == 0) atomic_done(atomicAdd(&R.tp[F.packets[k].tp], b));
     }
-    // the state is read above by every wave before the last workgroup to arrive replaces it
+    // The state is read above by every wave before the last workgroup to arrive replaces it; of
+    // the other workgroups' results that one reads R.tp alone, by atomics (atomic_done).
     __syncthreads();
     if (threadIdx.x == 0) s_last = atomicAdd(&R.arrived, 1u) == groups - 1;
     __syncthreads();
@@ -655,7 +659,7 @@ __global__ void __launch_bounds__(kHullThreads) rc_dist_kernel(RcParams P) {
     }
     unsigned long long* sums = P.dist + (size_t)f * kRcDistSums;
     atomic_done(atomicExch(&sums[t], __builtin_bit_cast(unsigned long long, dist)));
-    uint32_t last = 0;
+    uint32_t last = 0;  // reads the other workgroups' sums by atomics only (atomic_done)
     if (threadIdx.x == 0) last = atomicAdd(&P.runs[f].summed, 1u) == groups - 1;
     if (!__shfl((int)last, 0)) return;
     double s[groups];

@@ -181,8 +181,10 @@ GAIL_HD int rc_bin_of(double s, int64_t kLo, int nb, const unsigned long long* m
 
 // ---------------------------------------------------------------- packet headers
 // B.10.1 packet-header bits: bytes fill MSB first and a byte after 0xFF carries 7 bits, so no
-// marker can appear in a header. Each finished byte goes to `out` (RcCount drops it: the
-// device only needs the count; the host's Tier-2 writer appends it to the codestream).
+// marker can appear in a header. Each finished byte goes to `out` (RcCount drops it where only
+// the count is wanted; the Tier-2 writer appends it to the codestream). The code of this
+// section runs on the host; the device sizes packets with code of its own (measure_packet in
+// kernels_rc.hip), which must agree with it.
 struct RcCount {
     GAIL_HD void operator()(uint32_t) const {}
 };
@@ -254,9 +256,7 @@ template <class Sink> GAIL_HD void rc_pass_count(Sink& bw, int n) {
 //     value 1;
 //   zero bit-planes (coded to the end, included blocks only): a node not yet visited emits
 //     value - parent value zeros and a 1.
-// That is what the general tag-tree coder emits for these thresholds. Everything else
-// lives in registers (the leaves of a band are unrolled), so the device sizes a packet in
-// one thread without memory traffic beyond its blocks.
+// That is what the general tag-tree coder emits for these thresholds.
 template <class Blocks, class Sink, class Body>
 GAIL_HD bool rc_packet_code(const RcPacket& P, const RcPBand* pbands, const Blocks& blk, Sink& bw, const Body& body) {
     bw.bits(1, 1);
