@@ -122,6 +122,7 @@ struct HullSink {
 // A block's pass tables are rows of kMaxPasses entries: four at a time, the last four again
 // beyond the row's end.
 struct DevPassRows {
+    static constexpr int kGroup = 4;
     const uint4* len;
     const int4* dist;
     __device__ void load(int k, int, uint32_t* l, int32_t* d) const {

@@ -29,10 +29,11 @@ GAIL_HD double rc_plane_scale(int nbps, int k) {
 }
 
 // Lower convex hull of a block's (rate, distortion) points (rate_control.cpp:38-86): pass
-// gives its cumulative truncation lengths and per-pass distortion reductions four passes at a
-// time, scale is delta^2 * weight of its subband, stack keeps the hull's points (rate, passes
-// and distortion, 0 the origin) while it is built. Hands point j to out(j, point) and returns
-// the number of points; their slopes fall strictly (the first may be infinite).
+// gives its cumulative truncation lengths and per-pass distortion reductions, kGroup passes at a
+// time and one group ahead of use (the device, which waits for memory, takes four); scale is
+// delta^2 * weight of its subband, stack keeps the hull's points (rate, passes and distortion, 0
+// the origin) while it is built. Hands point j to out(j, point) and returns the number of points;
+// their slopes fall strictly (the first may be infinite).
 template <class Passes, class Stack, class Sink>
 GAIL_HD int rc_block_hull_to(int np, int nbps, double scale, const Passes& pass, Stack& stack, Sink& out) {
     int m = 0;
@@ -40,17 +41,18 @@ GAIL_HD int rc_block_hull_to(int np, int nbps, double scale, const Passes& pass,
     double D = 0, last = 0;  // and the slope that leads to it (m > 0)
     stack.put(0, 0, 0, 0.0);
     double acc = 0;
-    uint32_t len[4], nextLen[4];
-    int32_t dist[4], nextDist[4];
+    constexpr int G = Passes::kGroup;
+    uint32_t len[G], nextLen[G];
+    int32_t dist[G], nextDist[G];
     pass.load(0, np, nextLen, nextDist);
-    for (int k0 = 0; k0 < np; k0 += 4) {
-        for (int j = 0; j < 4; ++j) {
+    for (int k0 = 0; k0 < np; k0 += G) {
+        for (int j = 0; j < G; ++j) {
             len[j] = nextLen[j];
             dist[j] = nextDist[j];
         }
-        pass.load(k0 + 4, np, nextLen, nextDist);
+        pass.load(k0 + G, np, nextLen, nextDist);
 GAIL_UNROLL
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < G; ++j) {
             const int k = k0 + j;
             if (k >= np) break;
             acc += (double)dist[j] * rc_plane_scale(nbps, k) * scale;
@@ -97,13 +99,12 @@ struct RcPointArray {
     GAIL_HD void operator()(int j, const RcPoint& q) const { p[j] = q; }
 };
 struct RcPassRows {
+    static constexpr int kGroup = 1;
     const uint32_t* len;
     const int32_t* dist;
     GAIL_HD void load(int k, int np, uint32_t* l, int32_t* d) const {
-        for (int j = 0; j < 4; ++j) {  // the caller copies all four, also past the last pass
-            l[j] = k + j < np ? len[k + j] : 0u;
-            d[j] = k + j < np ? dist[k + j] : 0;
-        }
+        l[0] = k < np ? len[k] : 0u;
+        d[0] = k < np ? dist[k] : 0;
     }
 };
 struct RcHullStack {
