@@ -15,7 +15,7 @@ namespace gail_amd {
 
 namespace {
 
-// Bytes a wave may read past a codeword's end (less than a dword of its window).
+// Bytes read past a codeword's end (a lane's 16-byte window, aligned down to 8).
 constexpr size_t kBytePad = 64;
 // Length classes of the block ordering (bytes / 4, longer blocks share the top class).
 constexpr uint32_t kLenKeys = 4096;
@@ -57,7 +57,7 @@ Decoder::Decoder(int device, const Layout& L, int reduce, bool highBits)
     if (reduce < 0 || reduce > L.levels) throw std::runtime_error("more resolution levels left out than the stream has");
     try {
         hipCheck(hipSetDevice(dev_), "hipSetDevice");
-        DeviceContext::get(dev_);  // the kernels' tables
+        ctx_ = &DeviceContext::get(dev_);  // with the kernels' tables
         ws_.resize(L_.levels + 1);
         hs_.resize(L_.levels + 1);
         ws_[0] = L_.width;
@@ -135,7 +135,8 @@ void Decoder::ensureDescs(size_t n) {
     capDescs_ = cap;
 }
 
-void DescPlan::plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks) {
+void DescPlan::plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks, uint64_t total,
+                    uint64_t others, int cus) {
     // Coded blocks longest first (a counting sort over length classes).
     count.assign(kLenKeys + 1, 0u);
     size_t ncoded = 0;
@@ -149,10 +150,41 @@ void DescPlan::plan(const std::vector<int>& wanted, const uint8_t* coded, const 
     order.resize(ncoded);
     for (size_t k = 0; k < wanted.size(); ++k)
         if (coded[k]) order[count[key(blocks[wanted[k]].len)]++] = (uint32_t)wanted[k];
+    lanes = 1;
+    starts.clear();
+    if (order.empty()) return;
+    // A wave each, unless the device has much to do: a wave decodes a block three times as fast as
+    // a lane does, but lanes get up to twice as many bytes decoded in the same time. Either gives
+    // the same words. What counts is bytes in units of the longest block, which is as long as a
+    // frame of waves takes: lanes when this frame has 6 a compute unit (fewer do not fill the chip
+    // with lanes) and the device 78, with other decoders' bytes counted four times, as they also
+    // fill the time that lanes wait.
+    // Frames/s with waves and with lanes: 4K of 2.5 MB (7 units a CU), one decoder 399 and 160, two
+    // 474 and 353, four 478 and 506-546, eight 426 and 605-642; 7.9 MB (19), one 168 and 106, two 183
+    // and 224, eight 183 and 330; 22 MB (39), one 82 and 80, two 88 and 137, eight 88 and 184; 40 MB
+    // (97), one 55 and 67, eight 59 and 106; 2K of 5.6 MB (11), one 233 and 141, two 334 and 258,
+    // eight 343 and 366. A DCI frame of 1.3 MB (4) always has waves: eight decoders 770 and 745.
+    const uint64_t unit = (uint64_t)std::max(1u, blocks[order[0]].len) * (uint64_t)cus;
+    if (total < 6 * unit || total + 4 * others < 78 * unit) return;
+    // Up to kDecWaveLanes blocks a wave under a byte budget that spreads the frame over about six
+    // waves a compute unit (lanes that do different things take turns, so a wave runs about as
+    // long as the sum of its blocks). With four waves, with six and with eight: 22 MB, eight
+    // decoders 189, 189 and 172 frames/s; 7.9 MB, two decoders 190, 223 and 238.
+    const uint64_t budget = total / (6 * (uint64_t)cus);
+    lanes = (uint32_t)kDecWaveLanes;
+    uint64_t bytes = 0;
+    for (uint32_t k = 0; k < order.size(); ++k) {
+        const uint32_t len = blocks[order[k]].len;
+        if (starts.empty() || k - starts.back() == lanes || bytes + len > budget) {
+            starts.push_back(k);
+            bytes = 0;
+        }
+        bytes += len;
+    }
 }
 
 void DescPlan::pack(const Layout& L, const DecCode* blocks, DecBlock* out) const {
-    for (const uint32_t i : order) {
+    auto entry = [&](uint32_t i) {
         const DecCode& c = blocks[i];
         const CodeBlock& cb = L.cblks[i];
         const Subband& b = L.bands[cb.band];
@@ -163,15 +195,24 @@ void DescPlan::pack(const Layout& L, const DecCode* blocks, DecBlock* out) const
                  ((uint32_t)c.nbps << 12) | ((uint32_t)c.passes << 18);
         d.dst = (uint32_t)b.comp * (uint32_t)L.width * (uint32_t)L.height +
                 (uint32_t)(b.py0 + cb.y0) * (uint32_t)L.width + (uint32_t)(b.px0 + cb.x0);
-        *out++ = d;
+        return d;
+    };
+    if (lanes == 1) {
+        for (const uint32_t i : order) *out++ = entry(i);
+        return;
+    }
+    for (size_t w = 0; w < starts.size(); ++w) {
+        const size_t end = w + 1 < starts.size() ? starts[w + 1] : order.size();
+        for (size_t k = starts[w]; k < starts[w] + lanes; ++k)
+            *out++ = k < end ? entry(order[k]) : DecBlock{0, 0, 0, kDecEmpty};
     }
 }
 
-uint32_t Decoder::buildDescs(const uint8_t* coded, const DecCode* blocks) {
-    plan_.plan(wanted_, coded, blocks);
-    ensureDescs(plan_.order.size());
+uint32_t Decoder::buildDescs(const uint8_t* coded, const DecCode* blocks, uint64_t total, uint64_t others) {
+    plan_.plan(wanted_, coded, blocks, total, others, ctx_->computeUnits());
+    ensureDescs(plan_.size());
     plan_.pack(L_, blocks, hDescs_);
-    return (uint32_t)plan_.order.size();
+    return (uint32_t)plan_.size();
 }
 
 void queueDecode(const Layout& L, const Layout& frame, int reduce, bool highBits, const DecodeBuffers& b, hipStream_t s,
@@ -182,6 +223,7 @@ void queueDecode(const Layout& L, const Layout& frame, int reduce, bool highBits
     tp.bytes = b.bytes;
     tp.blocks = b.descs;
     tp.nblocks = b.nd;
+    tp.lanes = b.lanes;
     tp.words = b.words;
     tp.nwords = (uint32_t)(3 * npix);
     tp.stride = W;
@@ -270,11 +312,20 @@ void Decoder::decode(const Layout& frame, const uint8_t* data, size_t size, cons
     // Blocks decoded: of the resolutions kept, with passes, bit-planes the block coder carries
     // and bytes inside the codestream; the rest stay zero.
     std::vector<uint8_t> coded(wanted_.size());
+    uint64_t total = 0;
     for (size_t k = 0; k < wanted_.size(); ++k) {
         const DecCode& c = blocks[wanted_[k]];
         coded[k] = c.passes && c.nbps >= 1 && c.nbps <= 30 && (size_t)c.offset + c.len <= size;
+        total += coded[k] ? c.len : 0u;
     }
-    const uint32_t nd = buildDescs(coded.data(), blocks);
+    // this frame's bytes are under way from here to the return, however the call ends
+    struct Load {
+        std::atomic<uint64_t>& sum;
+        const uint64_t bytes, others;
+        Load(std::atomic<uint64_t>& s, uint64_t b) : sum(s), bytes(b), others(s.fetch_add(b)) {}
+        ~Load() { sum.fetch_sub(bytes); }
+    } load(ctx_->decodeLoad(), total);
+    const uint32_t nd = buildDescs(coded.data(), blocks, total, load.others);
     const Mem in = memKind(data), outKind = memKind(dst);
     const bool devOut = outKind == Mem::Device;
     // pinned pictures are written by DMA when their rows go forwards
@@ -298,6 +349,7 @@ void Decoder::decode(const Layout& frame, const uint8_t* data, size_t size, cons
     buf.bytes = dBytes_;
     buf.descs = dDescs_;
     buf.nd = nd;
+    buf.lanes = plan_.lanes;
     buf.words = dWords_;
     buf.plane[0] = dPlane_[0];
     buf.plane[1] = dPlane_[1];
@@ -420,8 +472,8 @@ void decodeNoAlloc(int device, const Layout& frame, int reduce, bool highBits, c
             wanted.push_back(i);
             coded.push_back(c.passes && c.nbps >= 1 && c.nbps <= 30 && (size_t)c.offset + c.len <= size);
         }
-    plan.plan(wanted, coded.data(), blocks);
-    const uint32_t nd = (uint32_t)plan.order.size();
+    plan.plan(wanted, coded.data(), blocks, 0, 0, 1);  // a wave each: one call at a time, 6,708 blocks at most
+    const uint32_t nd = (uint32_t)plan.size();
     if ((size_t)nd * sizeof(DecBlock) > kNoAllocTableBytes) throw std::runtime_error("Tier-1 table larger than its room");
     table.resize(nd);
     plan.pack(frame, blocks, table.data());
@@ -437,6 +489,7 @@ void decodeNoAlloc(int device, const Layout& frame, int reduce, bool highBits, c
     b.bytes = bytes;
     b.descs = descs;
     b.nd = nd;
+    b.lanes = plan.lanes;
     b.out = static_cast<uint8_t*>(dst);
     b.pitch = (int64_t)strideBytes;
 

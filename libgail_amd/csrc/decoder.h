@@ -20,27 +20,34 @@ struct DecCode {
     uint8_t passes, nbps, pad[2];
 };
 
+class DeviceContext;
+
 struct DecodeTimes {
     double t1 = 0, dwt = 0, color = 0, total = 0;  // ms; t1 includes the codestream upload
 };
 
 constexpr int kMaxDecLevels = 8;
 
-// The Tier-1 decode table of one frame: the blocks to decode, a wave each, longest first (they
-// start first, and a frame takes as long as its longest block).
+// The Tier-1 decode table of one frame: the blocks to decode, longest first (they start first, and
+// a frame takes as long as its longest block), a wave each or, under load, a lane each.
 struct DescPlan {
     std::vector<uint32_t> order, count;
-    // wanted: the layout's blocks of the resolutions kept; coded[k]: wanted[k] has data.
-    void plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks);
-    // Writes the table, order.size() entries, to out.
+    std::vector<uint32_t> starts;  // of the waves' blocks in order, when they have a lane each
+    uint32_t lanes = 1;            // entries per wave
+    // wanted: the layout's blocks of the resolutions kept; coded[k]: wanted[k] has data; total:
+    // bytes of those; others: bytes that other decoders have under way on the device.
+    void plan(const std::vector<int>& wanted, const uint8_t* coded, const DecCode* blocks, uint64_t total,
+              uint64_t others, int cus);
+    // Writes the table, size() entries, to out.
     void pack(const Layout& L, const DecCode* blocks, DecBlock* out) const;
+    size_t size() const { return lanes == 1 ? order.size() : starts.size() * lanes; }
 };
 
 // Device buffers of one frame's decode.
 struct DecodeBuffers {
     const uint8_t* bytes = nullptr;   // codestream, readable 64 bytes past its end
     const DecBlock* descs = nullptr;  // nd table entries
-    uint32_t nd = 0;
+    uint32_t nd = 0, lanes = 1;
     uint32_t* words = nullptr;        // 3 W x H reconstruction words, zero beforehand
     float* plane[2] = {nullptr, nullptr};  // 3 W x H floats each, the inverse DWT's ping-pong
     float* wave = nullptr;            // dequantised planes wanted (3 W x H floats), or null
@@ -95,9 +102,9 @@ private:
     void release();
     void ensureBytes(size_t n);
     void ensureDescs(size_t n);
-    // Writes the table of the blocks marked in coded[] (one flag per wanted block), longest
-    // first; returns its entries.
-    uint32_t buildDescs(const uint8_t* coded, const DecCode* blocks);
+    // Writes the table of the blocks marked in coded[] (one flag per wanted block), of total
+    // bytes, while other decoders have `others` under way; returns its entries.
+    uint32_t buildDescs(const uint8_t* coded, const DecCode* blocks, uint64_t total, uint64_t others);
 
     int dev_;
     Layout L_;
@@ -106,6 +113,7 @@ private:
     int outW_ = 0, outH_ = 0;
     std::vector<int> ws_, hs_, wanted_;
     DescPlan plan_;
+    DeviceContext* ctx_ = nullptr;
     hipStream_t stream_ = nullptr;
     hipEvent_t ev_[4] = {};
     uint32_t* dWords_ = nullptr;

@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -85,12 +86,15 @@ public:
     const uint16_t* octaveFirst() const { return octF_; }
     const DevRcTables& rcTables(const Layout& L);
     int computeUnits() const { return cus_; }
+    // Codeword bytes of the frames that decoders have under way on the device.
+    std::atomic<uint64_t>& decodeLoad() { return decodeLoad_; }
     std::string name() const { return name_; }
     std::string arch() const { return arch_; }
 
 private:
     explicit DeviceContext(int device);
     int dev_ = 0, cus_ = 0;
+    std::atomic<uint64_t> decodeLoad_{0};
     float* log2_ = nullptr;
     float* thr_ = nullptr;
     unsigned long long* octM_ = nullptr;

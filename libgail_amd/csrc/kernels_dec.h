@@ -7,18 +7,21 @@
 
 namespace gail_amd {
 
-// One code-block to decode.
+// One code-block to decode. Lanes left empty have dst == kDecEmpty.
 struct DecBlock {
     uint32_t off, len;  // the codeword within the codestream buffer
     uint32_t geom;      // (w - 1) | (h - 1) << 5 | orient << 10 | nbps << 12 | passes << 18
     uint32_t dst;       // word index of the block's top-left sample in the Mallat planes
 };
-constexpr int kDecWaves = 4;  // waves, a block each, per workgroup
+constexpr uint32_t kDecEmpty = 0xFFFFFFFFu;
+constexpr int kDecWaves = 4;       // waves per workgroup
+constexpr int kDecWaveLanes = 16;  // blocks of a wave that has one in each of its first lanes
 
 struct T1DecodeParams {
     const uint8_t* bytes;  // codestream, readable 64 bytes past its end
     const DecBlock* blocks;
-    uint32_t nblocks;
+    uint32_t nblocks;      // entries
+    uint32_t lanes;        // entries per wave: 1, a block by a whole wave, or kDecWaveLanes
     uint32_t* words;       // 3 Mallat planes of reconstruction words, zero beforehand
     uint32_t nwords;
     uint32_t stride;       // words per plane row (the frame width)

@@ -1,7 +1,8 @@
 // Decoder kernels for CDNA4 (gfx950, wave64).
 //
-// Tier-1: a wave per code-block, longest first (t1_decode_wave.h). The reconstruction words of a
-// block are stored once, over planes that were cleared for the blocks without data.
+// Tier-1: a wave per code-block, longest first (t1_decode_wave.h), which stores a block's
+// reconstruction words once, or under load a lane per block (t1_decode_block.h), which adds to
+// them. The planes are cleared beforehand, for the blocks without data too.
 //
 // Inverse DWT: one launch per level; a workgroup owns a TX x TY tile of the level's output
 // and all three components. It gathers the tile plus a 4-sample mirrored halo from the four
@@ -18,6 +19,7 @@
 #include <cstdint>
 
 #include "kernels_dec.h"
+#include "t1_decode_block.h"
 #include "t1_decode_wave.h"
 #include "t1_tables.h"
 
@@ -28,6 +30,8 @@ namespace {
 __constant__ uint32_t kDecNext[2 * kMqCoderStates];
 __constant__ uint32_t kDecInitial[4];
 __constant__ uint8_t kDecSign[256];
+__constant__ uint32_t kDecMq[47];
+__constant__ uint8_t kDecZc[4 * 128];
 
 // ISO/IEC 15444-1 Table F.4, rounded to float as the CPU reference rounds them.
 constexpr float kK = (float)1.230174104914001;
@@ -100,6 +104,65 @@ __global__ void __launch_bounds__(64 * kDecWaves) t1_decode_kernel(T1DecodeParam
     mq.src = P.bytes + d.off;
     mq.len = d.len;
     t1_decode_wave(mq, w, h, orient, nbps, passes, P.words + d.dst, P.stride, s_pack, s_sign);
+}
+
+// What a wave with a block in each of its first lanes keeps in LDS, at [entry][lane]: a bank per
+// lane, whatever row each lane is on.
+struct DecLanes {
+    uint32_t rows[4][32][kDecWaveLanes];
+    uint32_t ctx[19][kDecWaveLanes];
+};
+
+struct LaneState {
+    DecLanes* s;
+    const uint32_t* mq;   // Table C.2
+    const uint8_t* zct;   // Table D.1 of the block's orientation
+    uint32_t lane;
+    __device__ __forceinline__ void reset() {
+        for (uint32_t r = 0; r < 32u; ++r)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s->rows[t][r][lane] = 0u;
+        for (uint32_t c = 0; c < 19u; ++c) s->ctx[c][lane] = mq[t1d_initial_state(c)];
+    }
+    __device__ __forceinline__ uint32_t rows(int t, uint32_t r) const { return s->rows[t][r][lane]; }
+    __device__ __forceinline__ void set_rows(int t, uint32_t r, uint32_t v) { s->rows[t][r][lane] = v; }
+    __device__ __forceinline__ uint32_t ctx(uint32_t c) const { return s->ctx[c][lane]; }
+    __device__ __forceinline__ void set_ctx(uint32_t c, uint32_t v) { s->ctx[c][lane] = v; }
+    __device__ __forceinline__ uint32_t tab(uint32_t i) const { return mq[i]; }
+    __device__ __forceinline__ uint32_t zc(uint32_t code) const { return zct[code]; }
+};
+
+// A lane's words, added to as its samples are decoded: no lane waits for a read of its output.
+struct AtomicSink {
+    uint32_t* base;
+    uint32_t stride;
+    __device__ __forceinline__ void add(uint32_t i, uint32_t v) {
+        __hip_atomic_fetch_add(base + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+
+// For devices that several decoders keep busy with long codewords (DescPlan::plan): the sequential
+// decoder (t1_decode_block.h), a block in each of a wave's first 16 lanes. Lanes that are at the
+// same kind of decision share its instructions, which a wave per block cannot; each one's chain
+// takes three times as long. 22 MB 4K frames, eight decoders: 189 frames/s, 88 with a wave per
+// block. The states of 16 lanes take 9.4 KB, so 16 waves a CU fit (more lanes, fewer waves).
+__global__ void __launch_bounds__(64 * kDecWaves) t1_decode_lanes_kernel(T1DecodeParams P) {
+    __shared__ DecLanes s_lanes[kDecWaves];
+    __shared__ uint32_t s_mq[47];
+    __shared__ uint8_t s_zc[4 * 128];
+    const int t = threadIdx.x;
+    if (t < 47) s_mq[t] = kDecMq[t];
+    for (int i = t; i < 4 * 128; i += 64 * kDecWaves) s_zc[i] = kDecZc[i];
+    __syncthreads();
+    const uint32_t lane = (uint32_t)t & 63u, wave = (uint32_t)t >> 6;
+    const uint32_t at = (blockIdx.x * kDecWaves + wave) * kDecWaveLanes + lane;
+    if (lane >= kDecWaveLanes || at >= P.nblocks) return;
+    uint32_t w, h, orient, nbps, passes;
+    const DecBlock d = P.blocks[at];
+    if (d.dst == kDecEmpty || !block_fields(P, d, w, h, orient, nbps, passes)) return;
+    LaneState st{&s_lanes[wave], s_mq, s_zc + 128u * orient, lane};
+    AtomicSink out{P.words + d.dst, P.stride};
+    t1d_decode_block(st, P.bytes, d.off, d.len, w, h, nbps, passes, out);
 }
 
 // ---------------------------------------------------------------- inverse DWT
@@ -274,7 +337,13 @@ hipError_t dec_tables_init() {
     build_mq_coder_table(tab, initial, 15);
     uint8_t sign[256];
     build_sign_table(sign);
-    hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(kDecNext), tab, sizeof tab);
+    uint32_t mq[47];
+    build_mq_table(mq);
+    uint8_t zc[4 * 128];
+    build_zc_table(zc);
+    hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(kDecMq), mq, sizeof mq);
+    if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(kDecZc), zc, sizeof zc);
+    if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(kDecNext), tab, sizeof tab);
     if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(kDecInitial), initial, sizeof initial);
     return e != hipSuccess ? e : hipMemcpyToSymbol(HIP_SYMBOL(kDecSign), sign, sizeof sign);
 }
@@ -299,8 +368,11 @@ hipError_t launch_zero_words(uint32_t* p, size_t n, hipStream_t s) {
 
 hipError_t launch_t1_decode(const T1DecodeParams& p, hipStream_t s) {
     if (!p.nblocks) return hipSuccess;
-    const uint32_t groups = (p.nblocks + kDecWaves - 1) / kDecWaves;
-    hipLaunchKernelGGL(t1_decode_kernel, dim3(groups), dim3(64 * kDecWaves), 0, s, p);
+    const uint32_t per = (uint32_t)kDecWaves * p.lanes, groups = (p.nblocks + per - 1) / per;
+    if (p.lanes == 1)
+        hipLaunchKernelGGL(t1_decode_kernel, dim3(groups), dim3(64 * kDecWaves), 0, s, p);
+    else
+        hipLaunchKernelGGL(t1_decode_lanes_kernel, dim3(groups), dim3(64 * kDecWaves), 0, s, p);
     return hipGetLastError();
 }
 

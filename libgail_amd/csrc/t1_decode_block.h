@@ -1,7 +1,7 @@
 // EBCOT Tier-1 decoding of one code-block (ISO/IEC 15444-1 Annexes C.3 and D, no mode
-// switches), decision by decision in the standard's order. The tests' sequential form of what a
-// wave does on the GPU (t1_decode_wave.h), itself checked against the oracle's decoder. Test
-// infrastructure.
+// switches), decision by decision in the standard's order, written once for a lane of the GPU
+// (t1_decode_lanes_kernel) and for a host build that checks it against the CPU decoder and is
+// what the host build of the wave's arithmetic decoder (t1_wave_mq.h) is compared with.
 //
 // The block's state is four sets of 32 row masks (bit x = column x): significant, negative,
 // coded in this plane's significance pass, refined before. A stripe's six significance rows
@@ -23,19 +23,43 @@
 #pragma once
 #include <cstdint>
 
+#if defined(__HIPCC__)
+#define T1D_FN __host__ __device__ __forceinline__
+#else
+#define T1D_FN inline
+#endif
+
 namespace gail_amd {
 
 constexpr uint32_t kDecCtxRl = 17, kDecCtxUni = 18;
 
 // Table C.2 entry a context starts from (Table D.7): context 0 at state 4, run length at 3,
 // uniform at 46, the rest at 0.
-inline uint32_t t1d_initial_state(uint32_t cx) {
+T1D_FN uint32_t t1d_initial_state(uint32_t cx) {
     return cx == 0u ? 4u : (cx == kDecCtxRl ? 3u : (cx == kDecCtxUni ? 46u : 0u));
 }
 
-inline uint32_t t1d_popc(uint32_t v) { return (uint32_t)__builtin_popcount(v); }
-inline uint32_t t1d_lowest(uint32_t v) { return (uint32_t)__builtin_ctz(v); }  // lowest set bit's index, v != 0
-inline int t1d_clz(uint32_t v) { return __builtin_clz(v); }                     // v != 0
+T1D_FN uint32_t t1d_popc(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (uint32_t)__popc(v);
+#else
+    return (uint32_t)__builtin_popcount(v);
+#endif
+}
+T1D_FN uint32_t t1d_lowest(uint32_t v) {  // index of the lowest set bit, v != 0
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (uint32_t)(__ffs(v) - 1);
+#else
+    return (uint32_t)__builtin_ctz(v);
+#endif
+}
+T1D_FN int t1d_clz(uint32_t v) {  // v != 0
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __clz((int)v);
+#else
+    return __builtin_clz(v);
+#endif
+}
 
 // Sign coding (Table D.3) by k = 3 * (hc + 1) + (vc + 1), hc / vc the clamped horizontal
 // and vertical contributions: four bits each, (context - 9) | flip << 3.
@@ -51,15 +75,15 @@ struct MqDec {
     uint32_t A, C;
     int32_t CT;
 
-    inline uint64_t load8(uint32_t at) const { return *reinterpret_cast<const uint64_t*>(src + at); }
-    inline uint32_t byte(uint32_t a) const {
+    T1D_FN uint64_t load8(uint32_t at) const { return *reinterpret_cast<const uint64_t*>(src + at); }
+    T1D_FN uint32_t byte(uint32_t a) const {
         if (a >= end) return 0xFFu;
         const uint32_t k = a - base;
         return (uint32_t)((k < 8u ? cur : nxt) >> (8u * (k & 7u))) & 0xFFu;
     }
     // BYTEIN (C.3.4): after 0xFF the next byte brings 7 bits, and one above 0x8F is a marker,
     // which stays unread and feeds ones.
-    inline void bytein() {
+    T1D_FN void bytein() {
         const uint32_t b = byte(bp), b1 = byte(bp + 1u);
         if (b != 0xFFu) {
             ++bp;
@@ -80,7 +104,7 @@ struct MqDec {
         }
     }
     // INITDEC (C.3.5) for the codeword in src[start, start + len).
-    inline void init(const uint8_t* s, uint32_t start, uint32_t len) {
+    T1D_FN void init(const uint8_t* s, uint32_t start, uint32_t len) {
         src = s;
         bp = start;
         end = start + len;
@@ -95,14 +119,16 @@ struct MqDec {
     }
     // DECODE (C.3.2) with RENORMD (C.3.3) in context cx; a context state is its Table C.2
     // word (Qe | NMPS << 16 | NLPS << 22 | SWITCH << 28) with the MPS in bit 31.
-    template <class State> inline uint32_t decode(State& st, uint32_t cx) {
+    template <class State> T1D_FN uint32_t decode(State& st, uint32_t cx) {
         const uint32_t s = st.ctx(cx);
+        // both successor states, read before they are known to be needed so the table reads
+        // overlap the interval arithmetic instead of following it
         const uint32_t t_mps = st.tab((s >> 16) & 63u), t_lps = st.tab((s >> 22) & 63u);
         const uint32_t qe = s & 0xFFFFu, mps = s >> 31;
         A -= qe;
         // upper sub-interval: the MPS unless A < Qe (MPS exchange); lower: the LPS unless
         // A < Qe (LPS exchange). Without a renormalisation (the MPS with A >= 0x8000) the
-        // state is kept and the shift count below is 0.
+        // state is kept and the shift count below is 0, so lanes run the same instructions.
         const bool upper = (C >> 16) >= qe;
         const bool xchg = A < qe;
         const uint32_t d = upper != xchg ? mps : mps ^ 1u;
@@ -127,7 +153,7 @@ struct MqDec {
 
 // Zero-coding code of the sample in row k (0..3) of the stripe whose significance rows are
 // S[0] (above) .. S[5] (below), column x: h | v << 2 | d << 4 (counts).
-inline uint32_t t1d_zc_code(const uint32_t (&S)[6], int k, uint32_t x) {
+T1D_FN uint32_t t1d_zc_code(const uint32_t (&S)[6], int k, uint32_t x) {
     const uint32_t bit = 1u << x;
     const uint32_t side = (bit << 1) | (bit >> 1);  // columns x - 1 and x + 1
     const uint32_t h = t1d_popc(S[k + 1] & side);
@@ -139,7 +165,7 @@ inline uint32_t t1d_zc_code(const uint32_t (&S)[6], int k, uint32_t x) {
 // The sample (row k of the stripe, column x) is significant from plane p on: decode its
 // sign (D.3.2) and add 3 * 2^p with the sign to its word.
 template <class State, class Sink>
-inline void t1d_become_sig(MqDec& mq, State& st, Sink& out, uint32_t (&S)[6], uint32_t (&G)[6], int k, uint32_t x,
+T1D_FN void t1d_become_sig(MqDec& mq, State& st, Sink& out, uint32_t (&S)[6], uint32_t (&G)[6], int k, uint32_t x,
                            uint32_t p, uint32_t row_off) {
     const uint32_t bit = 1u << x;
     const uint32_t left = x ? bit >> 1 : 0u, right = bit << 1;  // right is 0 for x = 31
@@ -161,7 +187,7 @@ inline void t1d_become_sig(MqDec& mq, State& st, Sink& out, uint32_t (&S)[6], ui
 // Decodes the first `passes` coding passes of a w x h block (1..32 each) with nbps
 // magnitude bit-planes (1..30); passes past the last plane are not decoded.
 template <class State, class Sink>
-inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint32_t len, uint32_t w, uint32_t h,
+T1D_FN void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint32_t len, uint32_t w, uint32_t h,
                              uint32_t nbps, uint32_t passes, Sink& out) {
     if (w == 0u || h == 0u || w > 32u || h > 32u || nbps == 0u || nbps > 30u || passes == 0u) return;
     if (passes > 3u * nbps - 2u) passes = 3u * nbps - 2u;
@@ -177,6 +203,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
             uint32_t S[6], G[6], M[4];  // M: columns present in each row of the stripe
             S[0] = y0 ? st.rows(0, y0 - 1u) : 0u;
             G[0] = y0 ? st.rows(1, y0 - 1u) : 0u;
+#pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const bool in = (uint32_t)k < rows;
                 S[k + 1] = in ? st.rows(0, y0 + k) : 0u;
@@ -190,6 +217,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                 // D.3.1: insignificant samples with a significant neighbour
                 uint32_t V[4] = {0u, 0u, 0u, 0u};
                 uint32_t todo = 0u;
+#pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const uint32_t n = S[k] | S[k + 1] | S[k + 2];
                     todo |= (n | (n << 1) | (n >> 1)) & ~S[k + 1] & M[k];
@@ -198,6 +226,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                     const uint32_t x = t1d_lowest(todo);
                     const uint32_t bit = 1u << x;
                     todo &= ~bit;
+#pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (!(M[k] & bit) || (S[k + 1] & bit)) continue;
                         const uint32_t code = t1d_zc_code(S, k, x);
@@ -209,6 +238,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                         }
                     }
                 }
+#pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if ((uint32_t)k < rows) {
                         st.set_rows(0, y0 + k, S[k + 1]);
@@ -219,6 +249,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                 // D.3.3: samples significant before this plane's significance pass
                 uint32_t V[4], R[4];
                 uint32_t todo = 0u;
+#pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     V[k] = (uint32_t)k < rows ? st.rows(2, y0 + k) : 0u;
                     R[k] = (uint32_t)k < rows ? st.rows(3, y0 + k) : 0u;
@@ -228,6 +259,7 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                     const uint32_t x = t1d_lowest(todo);
                     const uint32_t bit = 1u << x;
                     todo &= ~bit;
+#pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (!(S[k + 1] & ~V[k] & bit)) continue;
                         const uint32_t cx = (R[k] & bit) ? 16u : (t1d_zc_code(S, k, x) ? 15u : 14u);
@@ -236,12 +268,14 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                         out.add(row_off + (uint32_t)k * out.stride + x, b ? (1u << p) : (0u - (1u << p)));
                     }
                 }
+#pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if ((uint32_t)k < rows) st.set_rows(3, y0 + k, R[k]);
             } else {
                 // D.3.4: every sample neither significant nor coded in this plane yet
                 uint32_t U[4];
                 uint32_t todo = 0u;
+#pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     U[k] = (uint32_t)k < rows ? ~S[k + 1] & ~st.rows(2, y0 + k) & M[k] : 0u;
                     todo |= U[k];
@@ -258,16 +292,19 @@ inline void t1d_decode_block(State& st, const uint8_t* src, uint32_t start, uint
                         if (!mq.decode(st, kDecCtxRl)) continue;
                         k0 = (int)(mq.decode(st, kDecCtxUni) << 1);
                         k0 |= (int)mq.decode(st, kDecCtxUni);
+#pragma unroll
                         for (int k = 0; k < 4; ++k)
                             if (k == k0) t1d_become_sig(mq, st, out, S, G, k, x, p, row_off);
                         ++k0;
                     }
+#pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (k < k0 || !(U[k] & bit)) continue;
                         if (mq.decode(st, st.zc(t1d_zc_code(S, k, x))))
                             t1d_become_sig(mq, st, out, S, G, k, x, p, row_off);
                     }
                 }
+#pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if ((uint32_t)k < rows) {
                         st.set_rows(0, y0 + k, S[k + 1]);

@@ -22,7 +22,7 @@
 #include <vector>
 
 #include "t1_cm_masks.h"
-#include "zc_table.h"
+#include "t1_tables.h"
 
 using namespace gail_amd;
 

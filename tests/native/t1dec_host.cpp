@@ -1,12 +1,12 @@
-// The tests' sequential Tier-1 decoder (t1_decode_block.h) as a library, so that it can be
-// checked against the oracle's decoder. It is what the host build of the GPU's arithmetic decoder
-// is compared with (wavemq_host.cpp). Test infrastructure: loaded by tests/ only.
+// Host build of the sequential per-block code (libgail_amd/csrc/t1_decode_block.h) for the CPU
+// tests: the source that a lane of the GPU runs, with plain arrays in place of LDS and plain
+// additions in place of atomic adds, so its words can be checked against the oracle's
+// decoder without a GPU. Test infrastructure: loaded by tests/ only.
 #include <cstring>
 #include <vector>
 
 #include "t1_decode_block.h"
 #include "t1_tables.h"
-#include "zc_table.h"
 
 using namespace gail_amd;
 
@@ -57,7 +57,7 @@ const Tables g_tab;
 
 extern "C" {
 
-// Decodes a codeword placed `start` bytes into a buffer that can be read past its end, and
+// Decodes a codeword placed `start` bytes into a buffer padded as the device buffer is, and
 // returns the words with row stride w. Returns 1 when the block wrote outside its 32 x 32
 // words, else 0.
 int host_t1_decode_words(const uint8_t* data, uint32_t len, uint32_t start, int w, int h, int orient, int nbps,

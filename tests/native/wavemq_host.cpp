@@ -14,7 +14,6 @@
 #include "t1_decode_block.h"
 #include "t1_tables.h"
 #include "t1_wave_mq.h"
-#include "zc_table.h"
 
 using namespace gail_amd;
 

@@ -1,6 +1,6 @@
 """The oracle's decoder (oracle.c: or_t1_decode_words, or_idwt97_2d_f32, or_decode_frame)
-pinned on the CPU, and the tests' sequential block decoder (tests/native/t1_decode_block.h, what the
-host build of the GPU's arithmetic decoder is compared with) checked against it:
+pinned on the CPU, and the host build of the code that a lane of the GPU decodes a block with checked
+against it (the wave's is in test_wave_mq_host.py):
 
 * against the compiled reference (oracle/_ref: t1_dec.cpp, dwt_cpu.cpp, cpu_decode_backend.cpp,
   codestream_parse.cpp, t2_parse.cpp), bit for bit, where it was built;
@@ -74,9 +74,8 @@ def test_t1_words_truncated_closed_form(oracle):
 
 
 def test_host_build_of_device_decoder_matches_oracle(oracle):
-    """The sequential block decoder (t1_decode_block.h; the GPU's own arithmetic decoder is in
-    test_wave_mq_host.py): every truncation point, codewords at every alignment of its 8-byte
-    window."""
+    """The sequential per-block code of the GPU's lane kernel (t1_decode_block.h) compiled for the
+    host: every truncation point, codewords at every alignment of the 8-byte window."""
     lib = _host_decoder()
     rng = np.random.default_rng(11)
     checked = 0
