@@ -547,7 +547,7 @@ __device__ bool search_step(const RcParams& P, uint32_t f, RcFrame& F, const uns
 // search's probes, one after the other. One 4K frame has some 600 packets, a wave each. With
 // one workgroup per frame for the whole search (a thread per packet's header, 26 blocks a
 // thread, a thread's chain of 16 probes) a search of three measurements took 615 us for one 4K
-// frame and 660 for 16; these launches with the finish and distortion kernels take 97 and 190.
+// frame and 660 for 16; these launches with the finish and distortion kernels take 109 and 197.
 // Frames with one budget take 3 or 4 measurements, those held by a component's cap 5 and more:
 // six launches, each 4 us when there is nothing left to do (24 us otherwise); further steps run
 // in rc_finish_kernel at 180 us each.

@@ -156,7 +156,7 @@ hipError_t launch_quant_debug(const T1Block* blocks, const T1Band* bands, const 
 }
 
 // ---------------------------------------------------------------- context modelling
-// Bound by vector issue: 0.86 vector instructions a cycle and CU at 16 4K frames, three waves
+// Bound by vector issue: 0.86-0.89 vector instructions a cycle and CU at 16 4K frames, three waves
 // a SIMD (the magnitudes and planes of a column need 168 registers), LDS busy 40 % of the time
 // with the symbols' byte stores. So instructions are what is saved: the quantiser and the
 // stores have no branches (a lane without a symbol stores to a junk byte), a symbol's bits are
